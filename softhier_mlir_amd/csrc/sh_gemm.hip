@@ -20,7 +20,8 @@
 // Workgroup -> tile order is XCD-aware: dispatch deals workgroups round-robin over the XCDs, so workgroup b
 // takes logical tile (b % X) * (tiles / X) + b / X and each XCD walks a contiguous run of row-major tiles
 // (shared X row panels stay in that XCD's L2).
-#include "sh_common.h"
+#include "sh_gemm_dev.h"
+#include "sh_gemm_small.h"
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -33,129 +34,8 @@
 
 namespace {
 
-constexpr int BK = 64;
-
-struct GemmArgs {
-    const uint16_t *x, *w;
-    uint16_t *z;
-    float *part;                 // split-K partials [splits][M][N] (fp32), or null
-    const void *bias;            // null, fp16 or fp32 row of N
-    const uint16_t *res;         // null or fp16 [M, ldr]
-    uint64_t ldx, ldw, ldz, ldr;
-    uint32_t M, N, K;
-    uint32_t kps;                // K per split (multiple of BK)
-    uint32_t tiles_m, tiles_n, splits;
-    uint32_t accumulate, bias_fp32, act;
-    uint32_t xcd_groups;         // > 1: XCD-aware block remap with this many XCDs (requires divisibility)
-    uint32_t group_m;            // > 1: tiles ordered in bands of this many tile rows, column by column within a band
-    const float *ln_stats;       // LayerNorm fold (or null): (mu, r) per row, fp32 [M][2], or ln_parts partials ...
-    const float *ln_c;           // ... and c per column (fp32 [N]); the fp32 bias row is then d
-    uint32_t ln_parts;           // > 0: ln_stats holds ln_parts (sum, M2) pairs of 32 columns per row (row_partials)
-    float ln_eps;                // ... and the statistics are formed with this eps
-    float *stats_out;            // or null: the (sum, M2) pairs of every 32 columns of each stored row, [M][N / 32]
-};
-
-// (mu, r = 1 / sqrt(var + eps)) of row gm for the LayerNorm fold: given (ln_parts == 0), or formed from the row's
-// ln_parts partials (s_b, M2_b) of 32 columns each (Chan, Golub and LeVeque, "Algorithms for computing the sample
-// variance", 1983): mu = sum s_b / n, M2 = sum_b (M2_b + 32 (s_b / 32 - mu)^2), var = M2 / n, n = 32 ln_parts,
-// sums in block order. Up to 32 partials (K <= 1024) of a 16-byte aligned array are loaded at once into registers,
-// 16 bytes per load (only the P / 2 loads the row has: the partials are re-read by every column tile, so their volume
-// is what this costs), and summed twice; more, or an array that is only 8-byte aligned, are read twice from memory
-// 8 bytes at a time (the same sums in the same order). Every consumer (register epilogues, split-K reduction) forms
-// the statistics with this one function.
-__device__ __forceinline__ float2 ln_row(const GemmArgs &a, uint32_t gm) {
-    if (a.ln_parts == 0) return ((const float2 *)a.ln_stats)[gm];
-    const uint32_t P = a.ln_parts;
-    const float2 *pp = (const float2 *)a.ln_stats + (uint64_t)gm * P;
-    const float inv_n = 1.f / (32.f * (float)P);
-    float s = 0.f, m2 = 0.f;
-    if (P <= 32 && P % 2 == 0 && ((uintptr_t)a.ln_stats & 15u) == 0) {
-        const uint32_t last = P / 2 - 1;             // wave-uniform: the branches below skip whole loads
-        float4 q[16];
-#pragma unroll
-        for (int h = 0; h < 16; ++h)
-            if ((uint32_t)h <= last) q[h] = ((const float4 *)pp)[h];
-#pragma unroll
-        for (int h = 0; h < 16; ++h)
-            if ((uint32_t)h <= last) s += q[h].x + q[h].z;
-        const float mu = s * inv_n;
-#pragma unroll
-        for (int h = 0; h < 16; ++h) {
-            if ((uint32_t)h > last) continue;
-            const float d0 = fmaf(q[h].x, 1.f / 32.f, -mu), d1 = fmaf(q[h].z, 1.f / 32.f, -mu);
-            m2 += fmaf(32.f * d0, d0, q[h].y) + fmaf(32.f * d1, d1, q[h].w);
-        }
-        return make_float2(mu, sh_fast_rsq(fmaf(m2, inv_n, a.ln_eps)));
-    }
-    for (uint32_t b = 0; b < P; b += 2) s += pp[b].x + (b + 1 < P ? pp[b + 1].x : 0.f);
-    const float mu = s * inv_n;
-    for (uint32_t b = 0; b < P; b += 2) {
-        const float2 q0 = pp[b], q1 = b + 1 < P ? pp[b + 1] : make_float2(32.f * mu, 0.f);
-        const float d0 = fmaf(q0.x, 1.f / 32.f, -mu), d1 = fmaf(q1.x, 1.f / 32.f, -mu);
-        m2 += fmaf(32.f * d0, d0, q0.y) + fmaf(32.f * d1, d1, q1.y);
-    }
-    return make_float2(mu, sh_fast_rsq(fmaf(m2, inv_n, a.ln_eps)));
-}
-
-// A wavefront's rows' fold factors (r and r mu of rows mrow + 32 i + r32), formed once at the start of a tile so
-// the loads overlap its first DMAs and the epilogue waits on nothing: lane l forms rows mrow + l + 64 k, and each
-// lane takes its rows' factors from those lanes.
-template <int FM>
-struct LnRows { float r[FM], rm[FM]; };
-template <int FM>
-__device__ __forceinline__ LnRows<FM> ln_rows(const GemmArgs &a, uint32_t mrow) {
-    constexpr int RPL = (FM + 1) / 2;                // rows formed per lane
-    LnRows<FM> l;
-    const int lane = threadIdx.x & 63, r32 = lane & 31;
-    if (!a.ln_stats) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i) { l.r[i] = 0.f; l.rm[i] = 0.f; }
-        return l;
-    }
-    float2 st[RPL];
-#pragma unroll
-    for (int k = 0; k < RPL; ++k) st[k] = ln_row(a, min(mrow + 64 * k + lane, a.M - 1));
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {                   // row 32 i + r32 was formed by lane 32 (i % 2) + r32, k = i / 2
-        const float mu = __shfl(st[i / 2].x, 32 * (i % 2) + r32, 64), r = __shfl(st[i / 2].y, 32 * (i % 2) + r32, 64);
-        l.r[i] = r;
-        l.rm[i] = mu * r;
-    }
-    return l;
-}
-
-// LayerNorm folded into the product (sh_gemm_epi.ln_stats): p -> r p - (r mu) c + d in fp32, before the fp16
-// rounding; the bias (d) is part of this step, so the chain below skips it. st = ln_row(a, gm).
-__device__ __forceinline__ float ln_apply(const GemmArgs &a, float2 st, float p, uint32_t gn) {
-    return fmaf(st.y, p, fmaf(-(st.x * st.y), a.ln_c[gn], ((const float *)a.bias)[gn]));
-}
-
-// Logical tile of block b -> (split, tile row, tile column). Dispatch deals workgroups round-robin over the
-// XCDs, so block b becomes logical index (b % X) (T / X) + b / X: each XCD walks a contiguous run of the tile
-// order and the operand panels it shares stay in that XCD's L2. The order is row-major, or (group_m > 1) in bands
-// of group_m tile rows taken column by column, so the tiles an XCD runs at once span group_m row panels of X and
-// a few column panels of W instead of every column panel (a bijection: a band's last, short one included).
-__device__ __forceinline__ void tile_of(const GemmArgs &a, uint32_t b, uint32_t nblk, uint32_t &tm, uint32_t &tn, uint32_t &split) {
-    uint32_t L = b;
-    if (a.xcd_groups > 1) L = (b % a.xcd_groups) * (nblk / a.xcd_groups) + b / a.xcd_groups;
-    const uint32_t per = a.tiles_m * a.tiles_n;
-    split = L / per;
-    const uint32_t l = L - split * per;
-    if (a.group_m > 1) {
-        const uint32_t band = l / (a.group_m * a.tiles_n), first = band * a.group_m;
-        const uint32_t rows = min(a.group_m, a.tiles_m - first), w = l - band * a.group_m * a.tiles_n;
-        tm = first + w % rows;
-        tn = w / rows;
-    } else {
-        tm = l / a.tiles_n;
-        tn = l % a.tiles_n;
-    }
-}
-
 // Zero-filled stand-in read by the epilogue for operands a call does not have (never written).
 __device__ __align__(64) uint32_t g_epi_zero[16];
-
-__device__ __forceinline__ uint32_t swz(uint32_t r) { return (r ^ (r >> 3)) & 7u; }
 
 template <int BM, int BN>
 struct Cfg {
@@ -166,8 +46,6 @@ struct Cfg {
     static constexpr size_t LDS = (2 * STAGE_BYTES > (size_t)BM * BN * 2) ? 2 * STAGE_BYTES : (size_t)BM * BN * 2;
     static_assert(BM % 64 == 0 && BN % 64 == 0 && BN <= 256 && BM * 8 % 256 == 0, "tile");
 };
-
-__device__ __forceinline__ uint4 zero4() { return make_uint4(0, 0, 0, 0); }
 
 // 8 halves starting at element (r, c) of a row-major [rows, ld] matrix, zero outside [0, rmax) x [0, cmax).
 template <bool VEC>
@@ -181,58 +59,6 @@ __device__ __forceinline__ uint4 load8(const uint16_t *p, uint64_t ld, uint32_t 
         for (int e = 0; e < 8; ++e) h[e] = (r < rmax && c + e < cmax) ? p[(uint64_t)r * ld + c + e] : 0u;
         return make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
     }
-}
-
-__device__ __forceinline__ uint32_t comp(const uint4 &q, int i) { return i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w; }
-
-// The epilogue chain applied to one fp16 product value, each step rounded to fp16 exactly as the unfused
-// library sequence sh_gemm -> (accumulate) -> sh_add_bias -> sh_gelu -> sh_add would store it:
-// z = r16(z_old + p) [accumulate]; z = r16(z + bias); z = r16(gelu(z)); z = r16(z + residual).
-__device__ __forceinline__ uint16_t epi_chain(const GemmArgs &a, uint16_t p, uint32_t gm, uint32_t gn) {
-    float v = sh_dev_h2f(p);
-    if (a.accumulate) v = sh_dev_h2f(sh_dev_f2h_rr(v + sh_dev_h2f(a.z[(uint64_t)gm * a.ldz + gn])));
-    if (a.bias && !a.ln_stats) {
-        const float b = a.bias_fp32 ? ((const float *)a.bias)[gn] : sh_dev_h2f(((const uint16_t *)a.bias)[gn]);
-        v = sh_dev_h2f(sh_dev_f2h_rr(v + b));
-    }
-    if (a.act == SH_ACT_GELU) { const uint16_t h = sh_dev_f2h(v); v = sh_dev_h2f((uint16_t)sh_gelu_u32(h | ((uint32_t)h << 16))); }
-    if (a.res) v += sh_dev_h2f(a.res[(uint64_t)gm * a.ldr + gn]);
-    return sh_dev_f2h(v);
-}
-
-// The same chain on 8 consecutive columns, with z_old / bias / residual already loaded (16-byte chunks; an
-// fp32 bias is b0:b1). fp16 + fp16 steps use packed fp16 adds, which round exactly like the fp32 form above.
-__device__ __forceinline__ uint4 epi_chain8(const GemmArgs &a, uint4 q, const uint4 &zo, const uint4 &b0, const uint4 &b1,
-                                            const uint4 &rq) {
-    uint32_t w[4] = {q.x, q.y, q.z, q.w};
-    if (a.accumulate) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) w[p] = sh_hadd2(comp(zo, p), w[p]);
-    }
-    if (a.bias && !a.ln_stats) {
-        if (a.bias_fp32) {
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const sh_h2 h = __builtin_bit_cast(sh_h2, w[p]);
-                const uint4 &bb = p < 2 ? b0 : b1;
-                const float lo = (float)h.x + __uint_as_float(comp(bb, (2 * p) & 3));
-                const float hi = (float)h.y + __uint_as_float(comp(bb, (2 * p + 1) & 3));
-                w[p] = (uint32_t)sh_dev_f2h_rr(lo) | ((uint32_t)sh_dev_f2h_rr(hi) << 16);
-            }
-        } else {
-#pragma unroll
-            for (int p = 0; p < 4; ++p) w[p] = sh_hadd2(w[p], comp(b0, p));
-        }
-    }
-    if (a.act == SH_ACT_GELU) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) w[p] = sh_gelu_u32(w[p]);
-    }
-    if (a.res) {
-#pragma unroll
-        for (int p = 0; p < 4; ++p) w[p] = sh_hadd2(w[p], comp(rq, p));
-    }
-    return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 // Accumulators -> Z. Element (i, j, r) of a wavefront is tile row wm*TM + 32 i + 8 (r/4) + 4 g + r%4 and
@@ -348,9 +174,8 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
     const int wm = wave >> 1, wn = wave & 1, g = lane >> 5, r32 = lane & 31;
 
     // workgroup -> (split, tile_m, tile_n)
-    const uint32_t nblk = a.tiles_m * a.tiles_n * a.splits;
     uint32_t tm, tn, split;
-    tile_of(a, blockIdx.x, nblk, tm, tn, split);
+    tile_of(a, blockIdx.x, tm, tn, split);
     const uint32_t m0 = tm * BM, n0 = tn * BN;
     const uint32_t kbeg = split * a.kps;
     const uint32_t kend = min(a.K, kbeg + a.kps);
@@ -479,11 +304,6 @@ struct Cfg2 {
     static_assert(LOADS < 64 && LDS <= 160 * 1024, "resources");
 };
 
-template <int BN>
-__device__ __forceinline__ uint32_t fw(uint32_t k) {
-    return ((BN / 8) % 16 == 0) ? 4u * (k & 3u) : 4u * ((k >> 1) & 1u);
-}
-
 template <int BM, int BN, int STAGES, bool SPLIT, bool KTAIL = false>
 __global__ __launch_bounds__(256) void k_gemm2(GemmArgs a) {
     using C = Cfg2<BM, BN, STAGES>;
@@ -491,9 +311,8 @@ __global__ __launch_bounds__(256) void k_gemm2(GemmArgs a) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wm = wave >> 1, wn = wave & 1, g = lane >> 5, r32 = lane & 31;
 
-    const uint32_t nblk = a.tiles_m * a.tiles_n * a.splits;
     uint32_t tm, tn, split;
-    tile_of(a, blockIdx.x, nblk, tm, tn, split);
+    tile_of(a, blockIdx.x, tm, tn, split);
     const uint32_t m0 = tm * BM, n0 = tn * BN;
     const uint32_t kbeg = split * a.kps;
     const uint32_t kend = min(a.K, kbeg + a.kps);
@@ -607,195 +426,6 @@ __global__ __launch_bounds__(256) void k_gemm2(GemmArgs a) {
     sh_wait_vmcnt<0>();     // the clamped tail loads must land before the tile is staged in the same LDS
     __syncthreads();     // every wavefront is done with the slices before the tile is staged in the same LDS
     epilogue<BM, BN, true, SPLIT, C::FM, C::FN>(a, acc, m0, n0, split, (uint16_t *)smem);
-}
-
-// ---- epilogue from registers (Z^T accumulator layout) ------------------------------------------------------
-// Kernels that pass the MFMA operands swapped (first = W fragment, second = X fragment) hold every 32 x 32
-// accumulator as a block of Z^T: lane l has row l % 32 of Z and columns 8 q + 4 g + e in register 4 q + e
-// (q, e = 0..3, g = l / 32). One permlane32 swap per register pair hands each lane 8 consecutive columns of its
-// row, which pass through the epilogue chain and leave as one 16-byte store: no LDS staging and no barrier.
-// The products are the same k-ordered sums as with the operands in X, W order (the tests check every
-// configuration stores the same bits). The helpers take the wavefront's position (wm, wn) in the 2 x 2 grid of
-// (BM/2) x (BN/2) sub-tiles.
-
-// x's upper 32 lanes <-> y's lower 32 lanes (v_permlane32_swap_b32).
-__device__ __forceinline__ void swap_halves(uint32_t &x, uint32_t &y) {
-    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-    x = r[0];
-    y = r[1];
-}
-
-__device__ __forceinline__ uint32_t pack_h2(float lo, float hi) {     // (fp32 values rounded to fp16 once more)
-    asm volatile("" : "+v"(lo), "+v"(hi));           // (as sh_dev_f2h_rr: no conversion folded into the producer)
-    return __builtin_bit_cast(uint32_t, sh_h2{(_Float16)lo, (_Float16)hi});
-}
-
-// The LayerNorm fold on a wavefront's Z^T accumulators (block (i, j) of lane l: the row of ln's entry i, columns
-// ncol + 32 j + 8 q + 4 g + e in register 4 q + e), in place, before they are rounded.
-template <int FM, int FN, bool OFF32 = false>
-__device__ __forceinline__ void ln_fold_zt(const GemmArgs &a, sh_f16v (&acc)[FM][FN], const LnRows<FM> &ln, uint32_t ncol) {
-    const int lane = threadIdx.x & 63, g = lane >> 5;
-    const float *rr = ln.r, *rm = ln.rm;
-    const float *d = (const float *)a.bias;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        float cj[16], dj[16];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t n = min(ncol + 32 * j + 8 * q + 4 * g, a.N - 4);
-            // (OFF32: scalar base plus a 32-bit byte offset, N < 2^24)
-            const float4 c4 = OFF32 ? *(const float4 *)((const char *)a.ln_c + n * 4u) : *(const float4 *)(a.ln_c + n);
-            const float4 d4 = OFF32 ? *(const float4 *)((const char *)d + n * 4u) : *(const float4 *)(d + n);
-            cj[4 * q] = c4.x; cj[4 * q + 1] = c4.y; cj[4 * q + 2] = c4.z; cj[4 * q + 3] = c4.w;
-            dj[4 * q] = d4.x; dj[4 * q + 1] = d4.y; dj[4 * q + 2] = d4.z; dj[4 * q + 3] = d4.w;
-        }
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(rr[i], acc[i][j][r], fmaf(-rm[i], cj[r], dj[r]));
-    }
-}
-
-// Row partials of a wavefront's finished chunks (Z^T layout: chunk (i, j, p) of a lane is row rbase + 32 i + r32,
-// columns cbase + 32 j + 16 p + 8 g): for each row and each 32-column block, the sum s of its 32 stored fp16 values
-// and M2 = sum (v - s / 32)^2 (two passes in fp32; lanes g = 0, 1 hold 16 values each), written as a float2 to
-// stats_out[row][block] (the consumer combines a row's blocks with ln_row). Stores the same bits in every
-// register-epilogue tile (the same 32 values, the same order).
-template <int FM, int FN, bool OFF32 = false>
-__device__ __forceinline__ void stats_zt(const GemmArgs &a, const uint4 (&q)[FM][FN][2], uint32_t rbase, uint32_t cbase) {
-    const int lane = threadIdx.x & 63, g = lane >> 5, r32 = lane & 31;
-    const uint32_t P = a.N / 32;
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const uint32_t row = rbase + 32 * i + r32;
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            float x[16], sum = 0.f;
-#pragma unroll
-            for (int p = 0; p < 2; ++p)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const sh_h2 h = __builtin_bit_cast(sh_h2, comp(q[i][j][p], w));
-                    x[8 * p + 2 * w] = (float)h.x;
-                    x[8 * p + 2 * w + 1] = (float)h.y;
-                }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) sum += x[e];
-            sum += __shfl_xor(sum, 32, 64);
-            const float mb = sum * (1.f / 32.f);
-            float m2 = 0.f;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) { const float d = x[e] - mb; m2 = fmaf(d, d, m2); }
-            m2 += __shfl_xor(m2, 32, 64);
-            const uint32_t col = cbase + 32 * j;
-            if (g == 0 && row < a.M && col < a.N) {
-                if constexpr (OFF32)           // (M N / 4 bytes of partials < 4 GiB: the launch checks it)
-                    *(float2 *)((char *)a.stats_out + (__umul24(row, P) + col / 32) * 8u) = make_float2(sum, m2);
-                else
-                    ((float2 *)a.stats_out)[(uint64_t)row * P + col / 32] = make_float2(sum, m2);
-            }
-        }
-    }
-}
-
-// 8 consecutive fp16 products of row block i, column block j, half p of one lane, in the Z^T layout above.
-// Both 16-byte chunks (p = 0, 1) of the 32 x 32 block come out of the same four swaps.
-template <int FM, int FN>
-__device__ __forceinline__ void zt_chunks(const sh_f16v (&acc)[FM][FN], int i, int j, uint4 (&q)[2]) {
-    uint32_t P[4][2];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        P[u][0] = pack_h2(acc[i][j][4 * u], acc[i][j][4 * u + 1]);
-        P[u][1] = pack_h2(acc[i][j][4 * u + 2], acc[i][j][4 * u + 3]);
-    }
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        swap_halves(P[2 * p][0], P[2 * p + 1][0]);
-        swap_halves(P[2 * p][1], P[2 * p + 1][1]);
-        q[p] = make_uint4(P[2 * p][0], P[2 * p][1], P[2 * p + 1][0], P[2 * p + 1][1]);
-    }
-}
-
-// The epilogue chain on a tile's chunks in place (q from zt_chunks of every block; chunk (i, j, p) of a lane is
-// row m0 + wm TM + 32 i + r32, columns n0 + wn TN + 32 j + 16 p + 8 g). Converting every accumulator first
-// halves the registers the epilogue holds. For the common chains (fp16 or no bias, optional residual) every
-// operand load of the tile is issued in one batch, so the epilogue waits for one memory latency.
-template <int BM, int BN, int FM, int FN>
-__device__ __forceinline__ void chain_chunks(const GemmArgs &a, uint4 (&q)[FM][FN][2], uint32_t m0, uint32_t n0, int wm, int wn) {
-    constexpr int TM = BM / 2, TN = BN / 2;
-    const int lane = threadIdx.x & 63, g = lane >> 5, r32 = lane & 31;
-    if (!a.accumulate && (!a.bias || a.ln_stats) && !a.res && a.act == SH_ACT_NONE) return;
-    if (!a.accumulate && (!(a.bias && a.bias_fp32) || a.ln_stats)) {
-        uint4 bq[FN][2];
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                const uint32_t gn = n0 + wn * TN + 32 * j + 16 * p + 8 * g, gc = min(gn, a.N - 8);
-                bq[j][p] = (a.bias && !a.ln_stats) ? *(const uint4 *)((const uint16_t *)a.bias + gc) : zero4();
-            }
-        uint4 rq[FM][FN][2];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const uint32_t gm = m0 + wm * TM + 32 * i + r32;
-            const uint64_t rowr = (uint64_t)min(gm, a.M - 1) * a.ldr;
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    const uint32_t gn = n0 + wn * TN + 32 * j + 16 * p + 8 * g, gc = min(gn, a.N - 8);
-                    rq[i][j][p] = a.res ? *(const uint4 *)(a.res + rowr + gc) : zero4();
-                }
-        }
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int p = 0; p < 2; ++p) q[i][j][p] = epi_chain8(a, q[i][j][p], zero4(), bq[j][p], zero4(), rq[i][j][p]);
-        return;
-    }
-    // z_old (accumulate) or a 32-byte fp32 bias per chunk: one (row block, column block) at a time
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const uint32_t gm = m0 + wm * TM + 32 * i + r32;
-        const uint32_t gmc = min(gm, a.M - 1);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            uint4 zo[2], b0[2], b1[2], rq[2];
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                const uint32_t gn = n0 + wn * TN + 32 * j + 16 * p + 8 * g, gc = min(gn, a.N - 8);
-                zo[p] = a.accumulate ? *(const uint4 *)(a.z + (uint64_t)gmc * a.ldz + gc) : zero4();
-                if (a.bias && a.bias_fp32) {
-                    b0[p] = *(const uint4 *)((const float *)a.bias + gc);
-                    b1[p] = *(const uint4 *)((const float *)a.bias + gc + 4);
-                } else {
-                    b0[p] = a.bias ? *(const uint4 *)((const uint16_t *)a.bias + gc) : zero4();
-                    b1[p] = zero4();
-                }
-                rq[p] = a.res ? *(const uint4 *)(a.res + (uint64_t)gmc * a.ldr + gc) : zero4();
-            }
-#pragma unroll
-            for (int p = 0; p < 2; ++p) q[i][j][p] = epi_chain8(a, q[i][j][p], zo[p], b0[p], b1[p], rq[p]);
-        }
-    }
-}
-
-// Store a finished tile's chunks (origin m0, n0).
-template <int BM, int BN, int FM, int FN>
-__device__ __forceinline__ void store_all(const GemmArgs &a, const uint4 (&q)[FM][FN][2], uint32_t m0, uint32_t n0, int wm, int wn) {
-    constexpr int TM = BM / 2, TN = BN / 2;
-    const int lane = threadIdx.x & 63, g = lane >> 5, r32 = lane & 31;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                const uint32_t gm = m0 + wm * TM + 32 * i + r32, gn = n0 + wn * TN + 32 * j + 16 * p + 8 * g;
-                if (gm < a.M && gn < a.N) *(uint4 *)(a.z + (uint64_t)gm * a.ldz + gn) = q[i][j][p];
-            }
 }
 
 // Store a wavefront's finished block (TM x TN at rbase, cbase) through LDS: 32 rows at a time, its Z^T chunks (chunk
@@ -960,7 +590,10 @@ __device__ __forceinline__ GemmArgs gemm_epi_spec(const GemmArgs &in) {
     return a;
 }
 
-template <int BM, int BN, int SK, int NST, bool WT, int MINW, bool SPLIT, bool PRE, int KG = 1, int EPI = EPI_ANY>
+// LATE (64 x 64 tiles: one 32 x 32 block per wavefront, small problems): the fold's row partials and its c / d rows are
+// requested behind the first slices and used after the k-loop, in group 0 only; at tile start their uncoalesced loads and
+// the combine held a 12-slice kernel up by 1 us.
+template <int BM, int BN, int SK, int NST, bool WT, int MINW, bool SPLIT, bool PRE, int KG = 1, int EPI = EPI_ANY, bool LATE = false>
 __global__ __launch_bounds__(256 * KG, MINW) void k_gemm5(GemmArgs a_in) {
     static_assert(EPI == EPI_ANY || (!SPLIT && KG == 1 && !WT), "epilogue builds are unsplit");
     const GemmArgs a = gemm_epi_spec<EPI>(a_in);
@@ -974,9 +607,8 @@ __global__ __launch_bounds__(256 * KG, MINW) void k_gemm5(GemmArgs a_in) {
     const int wm = wave >> 1, wn = wave & 1, g = lane >> 5, r32 = lane & 31;
     uint4 *const ring = smem + (size_t)grp * (C::LDS / 16);     // this group's stages
 
-    const uint32_t nblk = a.tiles_m * a.tiles_n * (KG > 1 ? 1u : a.splits);
     uint32_t tm, tn, split;
-    tile_of(a, blockIdx.x, nblk, tm, tn, split);
+    tile_of(a, blockIdx.x, tm, tn, split);
     if constexpr (KG > 1) split = (uint32_t)grp;
     const uint32_t m0 = tm * BM, n0 = tn * BN;
     const uint32_t kbeg = split * a.kps;
@@ -1138,7 +770,21 @@ __global__ __launch_bounds__(256 * KG, MINW) void k_gemm5(GemmArgs a_in) {
     // the rows' fold factors: their partials are loaded after the first DMAs, so the two latencies overlap (loads
     // complete in issue order, so the wait for the partials also sees those DMAs land)
     __builtin_amdgcn_sched_barrier(0);
-    const LnRows<FM> lnw = ln_rows<FM>(a, m0 + wm * TM);
+    static_assert(!LATE || (FM == 1 && FN == 1), "late fold operands");
+    LnRows<FM> lnw;
+    LnPair lnp;
+    float4 lc[LATE ? 4 : 1], ld[LATE ? 4 : 1];
+    if constexpr (!LATE) {
+        lnw = ln_rows<FM>(a, m0 + wm * TM);
+    } else if (a.ln_stats && grp == 0) {
+        ln_pair_load(a, min(m0 + wm * TM + r32, a.M - 1), lnp);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t n = min(n0 + wn * TN + 8 * e + 4 * g, a.N - 4);
+            lc[LATE ? e : 0] = *(const float4 *)(a.ln_c + n);
+            ld[LATE ? e : 0] = *(const float4 *)((const float *)a.bias + n);
+        }
+    }
     // slice kt, held in ring stage st = kt % NST, fixed at compile time: the loop below is unrolled by the ring's
     // stages, so every fragment read is a per-lane register plus an immediate offset (no vector add per read)
     auto slice = [&](int kt, auto stc) __attribute__((always_inline)) {
@@ -1211,7 +857,21 @@ __global__ __launch_bounds__(256 * KG, MINW) void k_gemm5(GemmArgs a_in) {
     if constexpr (SPLIT) {
         store_partials_zt<BM, BN, FM, FN>(a, acc, m0, n0, split, wm, wn);
     } else {
-        if (a.ln_stats) ln_fold_zt<FM, FN, OFF32>(a, acc, lnw, n0 + wn * TN);
+        if constexpr (LATE) {
+            if (a.ln_stats) {                        // (the expressions of ln_fold_zt)
+                const float2 st = ln_pair_form(a, min(m0 + wm * TM + r32, a.M - 1), lnp);
+                const float lr = st.y, lrm = st.x * st.y;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 cv = lc[LATE ? q : 0], dv = ld[LATE ? q : 0];
+                    const float cc[4] = {cv.x, cv.y, cv.z, cv.w}, dd[4] = {dv.x, dv.y, dv.z, dv.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[0][0][4 * q + e] = fmaf(lr, acc[0][0][4 * q + e], fmaf(-lrm, cc[e], dd[e]));
+                }
+            }
+        } else if (a.ln_stats) {
+            ln_fold_zt<FM, FN, OFF32>(a, acc, lnw, n0 + wn * TN);
+        }
         uint4 qc[FM][FN][2];
 #pragma unroll
         for (int i = 0; i < FM; ++i)
@@ -1289,9 +949,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void k_gemm6(GemmArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave / WGN, wn = wave % WGN, g = lane >> 5, r32 = lane & 31;
 
-    const uint32_t nblk = a.tiles_m * a.tiles_n * a.splits;
     uint32_t tm, tn, split;
-    tile_of(a, blockIdx.x, nblk, tm, tn, split);
+    tile_of(a, blockIdx.x, tm, tn, split);
     const uint32_t m0 = tm * BM, n0 = tn * BN;
     const uint32_t kbeg = split * a.kps;
     const uint32_t kend = min(a.K, kbeg + a.kps);
@@ -1808,6 +1467,7 @@ uint32_t grid_of(GemmArgs &a) {
     // (3.9 MB of operands at K = 768, inside its 4 MB L2) instead of 4 and every one (SH_GEMM_GROUP=1: row-major)
     static const int gm = env_int("SH_GEMM_GROUP", 8);
     a.group_m = gm > 1 ? (uint32_t)gm : 1;
+    set_tile_order(a, nblk);
     return nblk;
 }
 
@@ -1969,6 +1629,97 @@ float *scratch_ptr() {
     return (float *)p;
 }
 
+// Whether a call runs on the small-problem / any-alignment kernels (sh_gemm_small.hip) or the 64 x 64 direct-to-LDS tile
+// with late fold operands, and with how many K ranges per workgroup; tile -1: the tile table. Chosen by sizes and
+// alignment alone, so calls that differ in their epilogue only store the same product bits. The lines were measured on
+// MI355X in replayed graphs (us; fold / stats: with the LayerNorm fold from row partials / bias, residual, row partials):
+//  - up to one 32 x 32 tile per CU: four K ranges of at least 192 k (256 x 768 x 768: 4.5 against 5.2 for the 64 x 64 tile,
+//    fold 5.4 against 11.8, x 3072: 7.3 against 13.0, with stats 8.0 against 23.9; 50 x 720 x 2048: 5.4 against 9.2);
+//    eight where the tiles leave three quarters of the CUs idle. Above one tile per CU they lose (588 x 768: 6.1 against
+//    5.6).
+//  - up to one 64 x 32 tile per CU with a long K: the same with 64-row tiles.
+//  - up to two 64 x 64 tiles per CU: that tile (fold 588 x 2304 x 768: 9.6 against 12.9; 1024 x 2304 (576 tiles): level),
+//    with two K ranges from K = 1024 on while it is at most one per CU (1024 x 768 x 3072 with stats: 13.4 against 15.9
+//    with one range and 27.4 for the table).
+//  - operands without 16-byte alignment, and W^T with K % 64 != 0: never the table, whose element-wise kernels are 4 to
+//    10 times slower (4096 x 768 x 588: 13 against 83; 1000 x 777 x 588: 8 against 54).
+struct SmallPlan { int tile; uint32_t ranges, kps; };
+SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats, bool ln_reg) {
+    const SmallPlan none{-1, 0, 0};
+    const int force = env_int("SH_GEMM_SMALL", -1);      // tests: -2 = the table, >= 0 = that variant where it can run
+    if (force == -2 || r.K == 0 || env_int("SH_GEMM_CFG", -1) >= 0) return none;
+    if ((ln && !ln_reg) || r.ldx >= (1u << 23) || r.ldw >= (1u << 23)) return none;
+    const uint32_t wr = r.wt ? r.N : r.K, wc = r.wt ? r.K : r.N;
+    const bool any = !vec || !fast;                      // needs the any-alignment build
+    if (any && (ln || stats || r.ldx < 8 || r.ldw < 8 || (uint64_t)(r.M - 1) * r.ldx + r.K < 8 ||
+                (uint64_t)(wr - 1) * r.ldw + wc < 8)) return none;
+    const bool table_ok = vec && (fast || !r.wt);        // the table has a direct-to-LDS kernel for it
+    const uint64_t cus = sh_num_cus() > 0 ? (uint64_t)sh_num_cus() : 256;
+    const uint64_t t32 = (uint64_t)sh_cdiv(r.M, 32) * sh_cdiv(r.N, 32), t64x32 = (uint64_t)sh_cdiv(r.M, 64) * sh_cdiv(r.N, 32);
+    const uint64_t t64 = (uint64_t)sh_cdiv(r.M, 64) * sh_cdiv(r.N, 64);
+    if (r.splits > 1) {
+        // a caller's K ranges keep the partials workspace, but for the two equal ranges that run in one workgroup anyway
+        // (launch: the planned tile's family sets the bits)
+        const SplitK sk = split_k(r.K, r.splits);
+        if (sk.splits > 1) {
+            if (any || r.wt || sk.splits != 2 || 2 * sk.kps != r.K || env_int("SH_GEMM_KG", 1) == 0 ||
+                !g_cfgs[choose(r.M, r.N, r.K, vec, fast, 2, false, false).cfg].v2) return none;
+            return t32 <= cus ? SmallPlan{SMALL_RANGES_32, 2, sk.kps} : t64 <= cus ? SmallPlan{SMALL_DMA2, 1, sk.kps} : none;
+        }
+    }
+    const SplitK one = split_k(r.K, 1);
+    if (force >= 0) {
+        const SplitK sk = split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, 4)));
+        if (force == SMALL_RANGES_32 || (force == SMALL_RANGES_64 && !ln)) return {force, sk.splits, sk.kps};
+        if ((force == SMALL_64x64 || force == SMALL_128x64) && !ln && !stats && r.ldx >= 8 && r.ldw >= 8) return {force, 1, one.kps};
+        if (force == SMALL_DMA && fast && !r.wt) return {force, 1, one.kps};
+        if (force == SMALL_DMA2 && fast && !r.wt && r.K % 128 == 0) return {force, 1, r.K / 2};
+        return none;
+    }
+    if (t32 <= cus) {
+        const SplitK sk = split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, 4 * t32 <= cus ? 8 : 4)));
+        return {SMALL_RANGES_32, sk.splits, sk.kps};
+    }
+    if (t64x32 <= cus && !ln && (r.K >= 1024 || !table_ok)) {
+        const SplitK sk = split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, 4)));
+        return {SMALL_RANGES_64, sk.splits, sk.kps};
+    }
+    if (fast && !r.wt) {
+        if (t64 <= cus && r.K >= 1024 && r.K % 128 == 0) return {SMALL_DMA2, 1, r.K / 2};
+        if (t64 <= 2 * cus) return {SMALL_DMA, 1, one.kps};
+    }
+    if (!table_ok) return {t64 <= 2 * cus ? SMALL_64x64 : SMALL_128x64, 1, one.kps};
+    return none;
+}
+
+// The 64 x 64 direct-to-LDS tile of small problems (LATE builds of k_gemm5), one or two K ranges per workgroup.
+struct SmallDma { KernelFn fn; uint32_t threads; size_t lds; bool attr_set; };
+SmallDma g_small_dma[2] = {{k_gemm5<64, 64, 64, 3, false, 2, false, true, 1, EPI_ANY, true>, 256, Cfg5<64, 64, 64, 3, false>::LDS, false},
+                           {k_gemm5<64, 64, 64, 3, false, 1, false, true, 2, EPI_ANY, true>, 512, 2 * Cfg5<64, 64, 64, 3, false>::LDS, false}};
+template <typename SetEpi>
+int launch_small(const GemmReq &r, const SmallPlan &sp, bool any, SetEpi set_epi, const char *name) {
+    const sh_gemm_epi *e = r.epi;
+    GemmArgs a{};
+    a.x = (const uint16_t *)r.x; a.w = (const uint16_t *)r.w; a.z = (uint16_t *)r.z;
+    a.bias = e ? (const void *)e->bias : nullptr; a.res = e ? (const uint16_t *)e->residual : nullptr;
+    a.ldx = r.ldx; a.ldw = r.ldw; a.ldz = r.ldz; a.ldr = e ? e->ldr : 0;
+    a.M = r.M; a.N = r.N; a.K = r.K; a.kps = sp.kps; a.splits = 1;
+    a.accumulate = r.accumulate; a.bias_fp32 = (e && e->bias_fmt == SH_BIAS_FP32) ? 1 : 0; a.act = e ? e->act : 0;
+    set_epi(a);
+    if ((uint64_t)sh_cdiv(r.M, kSmallDims[sp.tile].bm) * sh_cdiv(r.N, kSmallDims[sp.tile].bn) > 0x7FFFFFFFull ||
+        sh_cdiv(std::min(r.M, r.N), 32) > 65535) { sh_set_error(-1, "[%s] problem too large", name); return -1; }
+    a.tiles_m = sh_cdiv(r.M, kSmallDims[sp.tile].bm); a.tiles_n = sh_cdiv(r.N, kSmallDims[sp.tile].bn);
+    if (sp.tile >= SMALL_ANY_TILES) {
+        SmallDma &d = g_small_dma[sp.tile - SMALL_DMA];
+        if (!d.attr_set) { (void)hipFuncSetAttribute((const void *)d.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)d.lds); d.attr_set = true; }
+        const uint32_t nblk = grid_of(a);
+        hipLaunchKernelGGL(d.fn, dim3(nblk), dim3(d.threads), d.lds, sh_stream(), a);
+        return sh_launch_ok(name) ? 0 : SH_EHIP;
+    }
+    sh_gemm_small_enqueue(a, (SmallTile)sp.tile, r.wt, any, sp.ranges, sh_stream());
+    return sh_launch_ok(name) ? 0 : SH_EHIP;
+}
+
 int launch(const GemmReq &r, const char *name) {
     if (r.M == 0 || r.N == 0) return 0;
     const sh_gemm_epi *e = r.epi;
@@ -1989,13 +1740,15 @@ int launch(const GemmReq &r, const char *name) {
     }
     const bool ln_reg = ln && fast && sh_aligned16(e->ln_c) && sh_aligned16(bias);
     const bool want_reg = (ln || stats) && fast && (!ln || ln_reg);
-    Plan p = choose(r.M, r.N, r.K, vec, fast, r.splits, r.wt, want_reg);
-    if (r.mesh) p.splits = 1;
     auto set_epi = [&](GemmArgs &t) {
         t.ln_stats = ln ? (const float *)e->ln_stats : nullptr; t.ln_c = ln ? (const float *)e->ln_c : nullptr;
         t.ln_parts = ln ? e->ln_parts : 0; t.ln_eps = ln ? e->ln_eps : 0.f;
         t.stats_out = stats ? (float *)e->stats_out : nullptr;
     };
+    const SmallPlan sp = small_plan(r, vec, fast, ln, stats, ln_reg);
+    if (sp.tile >= 0) return launch_small(r, sp, !fast, set_epi, name);
+    Plan p = choose(r.M, r.N, r.K, vec, fast, r.splits, r.wt, want_reg);
+    if (r.mesh) p.splits = 1;
     if (fast && p.splits == 1 && g_cfgs[p.cfg].v2 && !r.part && (!(ln || stats) || (want_reg && g_cfgs[p.cfg].reg))) {
         GemmArgs t{};
         t.x = (const uint16_t *)r.x; t.w = (const uint16_t *)r.w; t.bias = (const void *)bias;
