@@ -1,0 +1,82 @@
+"""Head widths and key-block splits of the attention kernels against the oracle: the one-pass kernel at every width it has a
+build for, on sequences that end inside, at and past a key block (64) and a query block (128), and the key-splitting kernel
+(short unmasked sequences of 64-wide heads, every token-masked head) at the edges of its 32-query items and of its
+wavefronts' key blocks."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import _KEEP, to_dev, to_np
+from oracle import refs
+from softhier_mlir_amd import data, shops
+
+pytestmark = pytest.mark.gpu
+A = shops.addr
+
+
+@pytest.mark.parametrize("dh", [32, 64, 72, 80, 96, 128])
+@pytest.mark.parametrize("S", [1, 63, 65, 129, 200, 580])
+def test_one_pass_widths(lib, gpu, S, dh):
+    """Packed q | k | v rows of two sequences; values in the last columns of V and K rows reach only their own head (a width
+    that is no multiple of 32 reads past a row inside the kernel): a NaN planted in the next head's V must not leak."""
+    import torch
+    B, H = 2, 3
+    D = H * dh
+    q, k, v = (data.normal((B * S, D), 70 + i) for i in range(3))
+    v[:, dh:2 * dh] = np.nan                                  # head 1's values: heads 0 and 2 must stay finite
+    X = to_dev(np.concatenate([q, k, v], 1))
+    O = torch.full((B * S, D + 8), 7.0, dtype=torch.float16, device="cuda")
+    rc = lib.sh_attention_batched(A(X), A(X, D), A(X, 2 * D), A(O), B, S, D, H, 3 * D, 3 * D, 3 * D, D + 8,
+                                  S * 3 * D, S * 3 * D, S * 3 * D, S * (D + 8), dh ** -0.5, 0)
+    assert rc == 0, shops.last_error()
+    o = to_np(O)
+    assert (o[:, D:] == 7.0).all()
+    for h in (0, 2):
+        c = slice(h * dh, (h + 1) * dh)
+        want = refs.attention_batched(q[:, c], k[:, c], v[:, c], B, 1, dh ** -0.5)
+        bad, err, _ = refs.close(o[:, c], want)
+        assert bad == 0, (h, err)
+    assert np.isnan(o[:, dh:2 * dh]).all()
+
+
+@pytest.mark.parametrize("S,H", [(132, 3), (192, 4), (196, 12), (257, 2), (512, 2), (1000, 4)])
+@pytest.mark.parametrize("scale", [0.125, -0.3, 2.0])
+def test_split_keys_unmasked(lib, gpu, S, H, scale):
+    D = 64 * H
+    q, k, v = (data.normal((S, D), 80 + i) for i in range(3))
+    import torch
+    O = torch.zeros((S, D), dtype=torch.float16, device="cuda")
+    rc = lib.sh_attention_batched(A(to_dev(q)), A(to_dev(k)), A(to_dev(v)), A(O), 1, S, D, H, D, D, D, D, 0, 0, 0, 0, scale, 0)
+    assert rc == 0, shops.last_error()
+    # against float64 (the oracle rounds its scores to fp16, which a scale of 2 makes visible): the numerators' fp16 rounding
+    # moves the weighted mean of V by at most 2^-11 max|v| in the sum and as much in its normalisation, the output's own
+    # rounding adds 2^-11 max|v|, and the fp32 exponents (|c s| < 256, 2^-24 relative) less than 2^-15: below 2^-9 max|v|
+    o, x64 = to_np(O).astype(np.float64), [t.astype(np.float64) for t in (q, k, v)]
+    for h in range(H):
+        c = slice(64 * h, 64 * (h + 1))
+        t = scale * (x64[0][:, c] @ x64[1][:, c].T)
+        p = np.exp(t - t.max(1, keepdims=True))
+        want = (p / p.sum(1, keepdims=True)) @ x64[2][:, c]
+        assert np.abs(o[:, c] - want).max() <= 2.0 ** -9 * np.abs(x64[2][:, c]).max(), h
+
+
+@pytest.mark.parametrize("dh", [32, 64, 72, 80, 96, 128])
+@pytest.mark.parametrize("S", [4, 36, 64, 68, 200])
+def test_split_keys_masked(lib, gpu, S, dh):
+    """Causal tokens, a token array one element into its buffer, padding queries (uniform) and a first block whose keys no
+    query of a later class order may see."""
+    import torch
+    H, Hkv = 4, 2
+    D, DKV = H * dh, Hkv * dh
+    q, k, v = data.normal((S, D), 91), data.normal((S, DKV), 92), data.normal((S, DKV), 93)
+    Q, K, V = to_dev(q), to_dev(k), to_dev(v)
+    down = np.arange(S, dtype=np.uint32)[::-1].copy()         # query i sees keys j >= i
+    mix = np.array([(j % 3) if j % 11 else refs.LLM_PAD for j in range(S)], np.uint32)
+    for tok in (refs.llm_tokens(S, "causal"), down, mix):
+        T = torch.from_numpy(np.concatenate([[0], tok]).astype(np.uint16).view(np.int16)).cuda()
+        _KEEP.append(T)
+        O = torch.zeros((S, D), dtype=torch.float16, device="cuda")
+        assert lib.sh_attention_gqa(A(Q), A(K), A(V), A(O), S, D, H, Hkv, D, DKV, DKV, D, 0.125, A(T, 1), shops.SH_ALL) == 0, shops.last_error()
+        bad, err, _ = refs.close(to_np(O), refs.attention_gqa(q, k, v, H, Hkv, tok))
+        assert bad == 0, err
