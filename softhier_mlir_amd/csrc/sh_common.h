@@ -131,6 +131,43 @@ __device__ __forceinline__ sh_s4 sh_ds_read_tr(uint32_t addr) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) sh_s4 *)(uintptr_t)addr);
 }
 
+// 16-byte accesses at 2-byte alignment: gfx950 global loads and stores take any alignment.
+typedef uint32_t sh_u4v __attribute__((ext_vector_type(4)));
+typedef sh_u4v sh_u4v_a2 __attribute__((aligned(2)));
+typedef uint32_t sh_u2v_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t sh_u1_a2 __attribute__((aligned(2)));
+__device__ __forceinline__ uint4 sh_ld16_any(const uint16_t *p) {
+    const sh_u4v q = *(const sh_u4v_a2 *)p;
+    return make_uint4(q.x, q.y, q.z, q.w);
+}
+// v shifted down by `sh` halves, halves nv .. 7 cleared (sh, nv <= 8).
+__device__ __forceinline__ uint4 sh_fix8(uint4 v, uint32_t sh, uint32_t nv) {
+    uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
+    if (sh & 4u) { lo = hi; hi = 0; }
+    const uint32_t s = (sh & 3u) * 16u;
+    if (s) { lo = (lo >> s) | (hi << (64u - s)); hi >>= s; }
+    const uint64_t one = ~0ull;
+    const uint64_t ml = nv >= 4 ? one : (1ull << (16 * nv)) - 1, mh = nv >= 8 ? one : nv <= 4 ? 0 : (1ull << (16 * (nv - 4))) - 1;
+    lo &= ml;
+    hi &= mh;
+    return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+// Halves [c, c + 8) of a row of n >= 8 halves (zeros past its end; nothing past it is read): a chunk that reaches past the
+// end is loaded from the row's last 8 halves and shifted. c < n.
+__device__ __forceinline__ uint4 sh_ld8_row(const uint16_t *row, uint32_t c, uint32_t n) {
+    const uint32_t at = min(c, n - 8u);
+    const uint4 v = sh_ld16_any(row + at);
+    return at == c ? v : sh_fix8(v, c - at, 8u - (c - at));
+}
+// The first n halves of v to p (n >= 8: all).
+__device__ __forceinline__ void sh_st8_any(uint16_t *p, uint4 v, uint32_t n) {
+    if (n >= 8) { *(sh_u4v_a2 *)p = (sh_u4v){v.x, v.y, v.z, v.w}; return; }
+    uint32_t a = v.x, b = v.y;
+    if (n & 4u) { *(sh_u2v_a2 *)p = (sh_u2v_a2){v.x, v.y}; p += 4; a = v.z; b = v.w; }
+    if (n & 2u) { *(sh_u1_a2 *)p = a; p += 2; a = b; }
+    if (n & 1u) *p = (uint16_t)a;
+}
+
 static inline bool sh_aligned16(uint64_t p) { return (p & 15u) == 0; }
 static inline uint32_t sh_cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 

@@ -16,30 +16,10 @@
 
 namespace {
 
-// 16 bytes at an address that is only 2-byte aligned (EDGE): gfx950 global loads and stores take any alignment.
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-typedef u4v u4v_a2 __attribute__((aligned(2)));
 template <bool EDGE>
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) {
-    if constexpr (EDGE) {
-        const u4v q = *(const u4v_a2 *)p;
-        return make_uint4(q.x, q.y, q.z, q.w);
-    } else {
-        return *(const uint4 *)p;
-    }
-}
-
-// v shifted down by `sh` halves, halves nv .. 7 cleared (sh, nv <= 8).
-__device__ __forceinline__ uint4 fix8(uint4 v, uint32_t sh, uint32_t nv) {
-    uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
-    if (sh & 4u) { lo = hi; hi = 0; }
-    const uint32_t s = (sh & 3u) * 16u;
-    if (s) { lo = (lo >> s) | (hi << (64u - s)); hi >>= s; }
-    const uint64_t one = ~0ull;
-    const uint64_t ml = nv >= 4 ? one : (1ull << (16 * nv)) - 1, mh = nv >= 8 ? one : nv <= 4 ? 0 : (1ull << (16 * (nv - 4))) - 1;
-    lo &= ml;
-    hi &= mh;
-    return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    if constexpr (EDGE) return sh_ld16_any(p);
+    else return *(const uint4 *)p;
 }
 
 // W slice swizzle ([K, N] layout): as fw, but a 32-column row (4 chunks) needs none (4 rows span the banks).
@@ -157,9 +137,9 @@ __global__ __launch_bounds__(KS && FM == 1 ? 512 : 256, KS ? 1 : 2) void k_gemm_
         if (EDGE && kt == KT - 1) {
             uint32_t sh, nv;
 #pragma unroll
-            for (int r = 0; r < XR; ++r) { (void)last_x(r, sh, nv); rx[u][r] = fix8(rx[u][r], sh, nv); }
+            for (int r = 0; r < XR; ++r) { (void)last_x(r, sh, nv); rx[u][r] = sh_fix8(rx[u][r], sh, nv); }
 #pragma unroll
-            for (int r = 0; r < WR; ++r) { (void)last_w(r, sh, nv); rw[u][r] = fix8(rw[u][r], sh, nv); }
+            for (int r = 0; r < WR; ++r) { (void)last_w(r, sh, nv); rw[u][r] = sh_fix8(rw[u][r], sh, nv); }
         }
 #pragma unroll
         for (int r = 0; r < XR; ++r) {
@@ -374,7 +354,7 @@ __global__ __launch_bounds__(KS && FM == 1 ? 512 : 256, KS ? 1 : 2) void k_gemm_
                         b1 = ld16<true>((const uint16_t *)((const float *)a.bias + gn + 4));
                     }
                     const uint4 v = epi_chain8(a, qc[i][0][p], zo[i][p], b0, b1, rq[i][p]);
-                    *(u4v_a2 *)z = (u4v){v.x, v.y, v.z, v.w};
+                    sh_st8_any(z, v, 8);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)

@@ -6,7 +6,8 @@
 //  - transpose: 128 x 128 tiles, 8 x 8 register transposes into a swizzled LDS tile, 16-byte row stores;
 //    pure 16-bit moves, so the result is bit-exact (NaN payloads included).
 // Rows wider than the register-resident limit (8192 columns) use a block-per-row loop kernel. Tensors
-// whose base, leading dim or width is not a multiple of 8 halves take element-wise variants.
+// whose base, leading dim or width is not a multiple of 8 halves take the same chunks through 2-byte aligned accesses;
+// rows of fewer than 8 columns one half per access.
 #include "sh_common.h"
 #include <algorithm>
 #include <cstdlib>
@@ -31,9 +32,12 @@ __device__ __forceinline__ uint4 pack8(const float *f) {
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Row layouts (the kernels' VEC): SCALAR one half per access (rows of fewer than 8 columns), ALIGNED 16-byte chunks, ANY the
+// same chunks at any base, leading dim and width (2-byte aligned accesses, the row's last chunk loaded from its end).
+enum { SCALAR = 0, ALIGNED = 1, ANY = 2 };
 // Element index of slot (u, i) of a lane: vector layout = 8 consecutive halves per chunk, chunks strided by
 // 64 lanes; scalar layout = one half per lane, strided by 64.
-template <bool VEC>
+template <int VEC>
 __device__ __forceinline__ uint32_t slot_col(int lane, int u, int i) {
     return VEC ? 8u * (uint32_t)(lane + 64 * u) + (uint32_t)i : (uint32_t)lane + 64u * (uint32_t)(8 * u + i);
 }
@@ -46,7 +50,6 @@ __device__ __forceinline__ void pin4(uint4 &q) { __asm__ volatile("" : "+v"(q.x)
 // 16-byte store; nt: nontemporal (streaming), used when the output is at least half the 256 MB Infinity Cache: with
 // its input it does not stay there, so no consumer could find it cached and plain stores only evict what it could
 // use (at 16x the encoder's rows, ~200 MB outputs: LayerNorm 5.7 against 5.5 TB/s, add_bias 6.0 against 5.6).
-typedef uint32_t sh_u4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void st16(void *p, uint4 v, bool nt) {
     if (nt) __builtin_nontemporal_store((sh_u4v){v.x, v.y, v.z, v.w}, (sh_u4v *)p);
     else *(uint4 *)p = v;
@@ -66,12 +69,23 @@ __device__ __forceinline__ uint4 ld16(const void *p) {
     }
 }
 
-template <int NCH>
+template <int NCH, int VEC>
 __device__ __forceinline__ void load_raw(const uint16_t *__restrict__ p, uint32_t cols, int lane, uint4 (&raw)[NCH]) {
 #pragma unroll
     for (int u = 0; u < NCH; ++u) {
-        const uint32_t c0 = slot_col<true>(lane, u, 0);
-        raw[u] = *(const uint4 *)(p + (c0 < cols ? c0 : 0u));
+        const uint32_t c0 = slot_col<VEC>(lane, u, 0), c = c0 < cols ? c0 : 0u;
+        raw[u] = VEC == ANY ? sh_ld16_any(p + min(c, cols - 8u)) : *(const uint4 *)(p + c);
+    }
+}
+// ANY: a row's last chunk, loaded from its end, into place.
+template <int NCH, int VEC>
+__device__ __forceinline__ void place_raw(uint4 (&raw)[NCH], uint32_t cols, int lane) {
+    if constexpr (VEC == ANY) {
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) {
+            const uint32_t c0 = slot_col<VEC>(lane, u, 0);
+            if (c0 < cols && c0 + 8u > cols) raw[u] = sh_fix8(raw[u], c0 + 8u - cols, cols - c0);
+        }
     }
 }
 
@@ -81,19 +95,20 @@ __device__ __forceinline__ void unpack_row(const uint4 (&raw)[NCH], uint32_t col
     for (int u = 0; u < NCH; ++u) {
         float f[8];
         unpack8(raw[u], f);
-        const bool ok = slot_col<true>(lane, u, 0) < cols;
+        const bool ok = slot_col<ALIGNED>(lane, u, 0) < cols;
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[u][i] = ok ? f[i] : 0.f;
     }
 }
 
-template <int NCH, bool VEC>
+template <int NCH, int VEC>
 __device__ __forceinline__ void load_row(const uint16_t *__restrict__ p, uint32_t cols, int lane, float (&v)[NCH][8]) {
     if (VEC) {
         uint4 raw[NCH];
-        load_raw<NCH>(p, cols, lane, raw);
+        load_raw<NCH, VEC>(p, cols, lane, raw);
 #pragma unroll
         for (int u = 0; u < NCH; ++u) pin4(raw[u]);   // all chunks issued before the first wait
+        place_raw<NCH, VEC>(raw, cols, lane);
         unpack_row<NCH>(raw, cols, lane, v);
         return;
     }
@@ -101,22 +116,24 @@ __device__ __forceinline__ void load_row(const uint16_t *__restrict__ p, uint32_
     for (int u = 0; u < NCH; ++u)
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const uint32_t c = slot_col<false>(lane, u, i);
+            const uint32_t c = slot_col<SCALAR>(lane, u, i);
             v[u][i] = c < cols ? sh_dev_h2f(p[c]) : 0.f;
         }
 }
 
-template <int NCH, bool VEC>
+template <int NCH, int VEC>
 __device__ __forceinline__ void store_row(uint16_t *__restrict__ p, uint32_t cols, int lane, const float (&v)[NCH][8]) {
 #pragma unroll
     for (int u = 0; u < NCH; ++u) {
         if (VEC) {
-            const uint32_t c0 = slot_col<true>(lane, u, 0);
-            if (c0 < cols) *(uint4 *)(p + c0) = pack8(v[u]);
+            const uint32_t c0 = slot_col<VEC>(lane, u, 0);
+            if (c0 >= cols) continue;
+            if (VEC == ANY) sh_st8_any(p + c0, pack8(v[u]), cols - c0);
+            else *(uint4 *)(p + c0) = pack8(v[u]);
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const uint32_t c = slot_col<false>(lane, u, i);
+                const uint32_t c = slot_col<SCALAR>(lane, u, i);
                 if (c < cols) p[c] = sh_dev_f2h(v[u][i]);
             }
         }
@@ -124,7 +141,7 @@ __device__ __forceinline__ void store_row(uint16_t *__restrict__ p, uint32_t col
 }
 
 // y = (x - mean) rsqrt(var + eps) gamma + beta per row (biased variance, two-pass over registers).
-template <int NCH, bool VEC>
+template <int NCH, int VEC>
 __global__ __launch_bounds__(256) void k_layernorm(uint16_t *y, const uint16_t *x, const uint16_t *gamma, const uint16_t *beta,
                                                    uint32_t rows, uint32_t cols, uint64_t ldy, uint64_t ldx, float eps) {
     const int lane = threadIdx.x & 63;
@@ -133,15 +150,18 @@ __global__ __launch_bounds__(256) void k_layernorm(uint16_t *y, const uint16_t *
     float v[NCH][8], g[NCH][8], b[NCH][8];
     if (VEC) {                                        // x, gamma and beta loads in flight together
         uint4 rx[NCH], rg[NCH], rb[NCH];
-        load_raw<NCH>(x + row * ldx, cols, lane, rx);
-        load_raw<NCH>(gamma, cols, lane, rg);
-        load_raw<NCH>(beta, cols, lane, rb);
+        load_raw<NCH, VEC>(x + row * ldx, cols, lane, rx);
+        load_raw<NCH, VEC>(gamma, cols, lane, rg);
+        load_raw<NCH, VEC>(beta, cols, lane, rb);
 #pragma unroll
         for (int u = 0; u < NCH; ++u) {               // pin all three here: the compiler would otherwise sink
             pin4(rx[u]);                              // the gamma / beta loads past the reductions
             pin4(rg[u]);
             pin4(rb[u]);
         }
+        place_raw<NCH, VEC>(rx, cols, lane);
+        place_raw<NCH, VEC>(rg, cols, lane);
+        place_raw<NCH, VEC>(rb, cols, lane);
         unpack_row<NCH>(rx, cols, lane, v);
         unpack_row<NCH>(rg, cols, lane, g);
         unpack_row<NCH>(rb, cols, lane, b);
@@ -330,7 +350,7 @@ __global__ __launch_bounds__(256) void k_copy1(uint8_t *dst, const uint8_t *src,
 }
 
 // y = softmax(scale x) per row: exp(scale x - max) = 2^(c x - m), c = scale log2(e), m = max(c x).
-template <int NCH, bool VEC>
+template <int NCH, int VEC>
 __global__ __launch_bounds__(256) void k_softmax(uint16_t *y, const uint16_t *x, uint32_t rows, uint32_t cols, uint64_t ld, float c) {
     const int lane = threadIdx.x & 63;
     const uint32_t row = blockIdx.x * kRowWaves + (threadIdx.x >> 6);
@@ -531,8 +551,75 @@ __global__ __launch_bounds__(256) void k_elementwise(uint16_t *y, const uint16_t
     }
 }
 
+// Any base, leading dim and width of at least 8: chunks of 8 halves through 2-byte aligned 16-byte accesses, per row, or
+// (FLAT: ld == cols) of the whole tensor as one row, so only its last chunk can be short (a bias chunk may then span two
+// rows). A short chunk is loaded from the row's end; each item writes its own elements only, so y may alias an input.
+template <int OP, int U, bool FLAT>
+__global__ __launch_bounds__(256) void k_elementwise_any(uint16_t *y, const uint16_t *a, const uint16_t *b, uint32_t cols, ShDiv per_row,
+                                                         ShDiv by_cols, uint64_t ld, float s, uint32_t items, uint32_t total) {
+    const uint32_t base = blockIdx.x * (256u * U) + threadIdx.x;
+    uint4 ra[U], rb[U];
+    uint64_t off[U];
+    uint32_t n[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t it = base + u * 256u, itc = it < items ? it : 0u;
+        uint32_t c;                                      // column of the chunk's first element
+        if (FLAT) {
+            off[u] = 8ull * itc;
+            n[u] = total - 8u * itc;
+            c = OP == OP_BIAS ? 8u * itc - sh_div(8u * itc, by_cols) * cols : 0u;
+        } else {
+            const uint32_t r = sh_div(itc, per_row);
+            c = 8u * (itc - r * per_row.d);
+            off[u] = r * ld + c;
+            n[u] = cols - c;
+        }
+        const uint32_t back = n[u] < 8u ? 8u - n[u] : 0u;
+        ra[u] = sh_ld16_any(a + off[u] - back);
+        if (OP == OP_ADD || OP == OP_SILU_MUL) rb[u] = sh_ld16_any(b + off[u] - back);
+        else if (OP == OP_BIAS) rb[u] = sh_ld16_any(b + min(c, cols - 8u));
+        else rb[u] = make_uint4(0, 0, 0, 0);
+        if (back) {
+            ra[u] = sh_fix8(ra[u], back, n[u]);
+            if (OP == OP_ADD || OP == OP_SILU_MUL) rb[u] = sh_fix8(rb[u], back, n[u]);
+        }
+        if (OP == OP_BIAS && c + 8u > cols) {
+            rb[u] = sh_fix8(rb[u], c + 8u - cols, cols - c);
+            if (FLAT) {                                  // ... and the first columns of the next row
+                const uint32_t k = cols - c;             // halves k .. 7 = bias 0 .. 7 - k
+                uint32_t w[4] = {rb[u].x, rb[u].y, rb[u].z, rb[u].w};
+                for (uint32_t e = k; e < 8u; ++e) {
+                    const uint32_t v = (uint32_t)b[e - k] << (16 * (e & 1));
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) w[q] |= q == (int)(e >> 1) ? v : 0u;
+                }
+                rb[u] = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+        if (it >= items) n[u] = 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (n[u] == 0) continue;
+        uint4 o;
+        if (OP == OP_GELU) {
+            o = make_uint4(sh_gelu_u32(ra[u].x), sh_gelu_u32(ra[u].y), sh_gelu_u32(ra[u].z), sh_gelu_u32(ra[u].w));
+        } else {
+            float fa[8], fb[8];
+            unpack8(ra[u], fa);
+            unpack8(rb[u], fb);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) fa[i] = ew<OP>(fa[i], fb[i], s);
+            o = pack8(fa);
+        }
+        sh_st8_any(y + off[u], o, n[u]);
+    }
+}
+
 // dst[cols, rows] = src[rows, cols]^T, 128 x 128 tile per block, 8 x 8 blocks per thread.
-template <bool NT>
+// ANYA: any base, leading dim, row count and width of at least 8 (2-byte aligned accesses; short chunks at the edges).
+template <bool NT, bool ANYA = false>
 __global__ __launch_bounds__(256) void k_transpose8(uint16_t *dst, const uint16_t *src, uint32_t rows, uint32_t cols,
                                                     uint64_t lds, uint64_t ldd) {
     __shared__ uint4 tile[128 * 16];                      // [dst row local][16-byte chunk ^ swizzle]
@@ -540,11 +627,11 @@ __global__ __launch_bounds__(256) void k_transpose8(uint16_t *dst, const uint16_
     const uint32_t tr = blockIdx.y * 128u, tc = blockIdx.x * 128u;
     const int br = t >> 4, bc = t & 15;
     const uint32_t r0 = tr + 8u * br, c0 = tc + 8u * bc;
-    if (r0 < rows && c0 < cols) {                         // rows % 8 == cols % 8 == 0: blocks are whole
+    if (r0 < rows && c0 < cols) {                         // (aligned: rows % 8 == cols % 8 == 0, blocks are whole)
         uint32_t w[8][4];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const uint4 q = ld16<NT>(src + (uint64_t)(r0 + i) * lds + c0);
+            const uint4 q = ANYA ? sh_ld8_row(src + (uint64_t)min(r0 + i, rows - 1) * lds, c0, cols) : ld16<NT>(src + (uint64_t)(r0 + i) * lds + c0);
             w[i][0] = q.x; w[i][1] = q.y; w[i][2] = q.z; w[i][3] = q.w;
         }
 #pragma unroll
@@ -565,11 +652,13 @@ __global__ __launch_bounds__(256) void k_transpose8(uint16_t *dst, const uint16_
     for (int k = 0; k < 8; ++k) {
         const int R = (t >> 4) + 16 * k;
         const uint32_t drow = tc + R, dcol = tr + 8u * C;
-        if (drow < cols && dcol < rows) st16(dst + (uint64_t)drow * ldd + dcol, tile[R * 16 + (C ^ ((R >> 3) & 15))], NT);
+        if (ANYA) {
+            if (drow < cols && dcol < rows) sh_st8_any(dst + (uint64_t)drow * ldd + dcol, tile[R * 16 + (C ^ ((R >> 3) & 15))], rows - dcol);
+        } else if (drow < cols && dcol < rows) st16(dst + (uint64_t)drow * ldd + dcol, tile[R * 16 + (C ^ ((R >> 3) & 15))], NT);
     }
 }
 
-// Any shape / alignment: 32 x 32 tiles through LDS, one half per access.
+// Fewer than 8 rows or columns: 32 x 32 tiles through LDS, one half per access.
 __global__ __launch_bounds__(256) void k_transpose1(uint16_t *dst, const uint16_t *src, uint32_t rows, uint32_t cols,
                                                     uint64_t lds, uint64_t ldd) {
     __shared__ uint16_t tile[32][33];
@@ -629,8 +718,9 @@ void launch_layernorm(uint64_t y, uint64_t x, uint64_t g, uint64_t b, uint32_t r
         return;
     }
     const dim3 grid(sh_cdiv(rows, kRowWaves)), block(256);
-#define SH_LN(N) do { if (vec) hipLaunchKernelGGL((k_layernorm<N, true>), grid, block, 0, st, Y, X, G, B, rows, cols, (uint64_t)ldy, (uint64_t)ldx, eps); \
-                      else hipLaunchKernelGGL((k_layernorm<N, false>), grid, block, 0, st, Y, X, G, B, rows, cols, (uint64_t)ldy, (uint64_t)ldx, eps); } while (0)
+#define SH_LN(N) do { if (vec) hipLaunchKernelGGL((k_layernorm<N, ALIGNED>), grid, block, 0, st, Y, X, G, B, rows, cols, (uint64_t)ldy, (uint64_t)ldx, eps); \
+                      else if (cols >= 8) hipLaunchKernelGGL((k_layernorm<N, ANY>), grid, block, 0, st, Y, X, G, B, rows, cols, (uint64_t)ldy, (uint64_t)ldx, eps); \
+                      else hipLaunchKernelGGL((k_layernorm<1, SCALAR>), grid, block, 0, st, Y, X, G, B, rows, cols, (uint64_t)ldy, (uint64_t)ldx, eps); } while (0)
     if (cols <= 512) SH_LN(1); else if (cols <= 1024) SH_LN(2); else if (cols <= 2048) SH_LN(4); else if (cols <= 4096) SH_LN(8); else SH_LN(16);
 #undef SH_LN
     sh_launch_ok("sh_layernorm");
@@ -638,6 +728,41 @@ void launch_layernorm(uint64_t y, uint64_t x, uint64_t g, uint64_t b, uint32_t r
 
 void launch_elementwise(int op, uint64_t y, uint64_t a, uint64_t b, uint32_t rows, uint32_t cols, uint32_t ld, float s, const char *name) {
     hipStream_t st = sh_stream();
+    if (cols >= 8 && !vec_ok(cols, {y, a, b}, {ld})) {
+        // Odd widths or bases. A dense tensor is one row of rows x cols elements: the aligned kernel where that length and
+        // the bases allow it, else (and for any leading dim) the any-alignment one ([2999 x 1001]: GELU 6.5, add 5.7,
+        // add_bias 4.5, scale 4.3 us with one half per access)
+        const uint64_t total = (uint64_t)rows * cols;
+        const bool flat = (ld == cols || rows == 1) && total < (1ull << 32) - 8;
+        if (flat && op != OP_BIAS && total % 8 == 0 && vec_ok(8, {y, a, b}, {})) {
+            cols = (uint32_t)total;
+            ld = (uint32_t)total;
+            rows = 1;
+        } else {
+            const uint32_t pr = sh_cdiv(cols, 8);
+            const uint64_t items64 = flat ? (total + 7) / 8 : (uint64_t)rows * pr;
+            if (items64 > 0xFFFFFFFFull - 4096) { sh_set_error(-1, "[%s] %u x %u is too large", name, rows, cols); return; }
+            const uint32_t items = (uint32_t)items64;
+            const bool one = op == OP_GELU || total * 2 >= kNtBytes;
+            const dim3 grid(sh_cdiv(items, 256u * (one ? 1u : 4u))), block(256);
+            uint16_t *Y = (uint16_t *)y; const uint16_t *A = (const uint16_t *)a, *B = (const uint16_t *)b;
+            const ShDiv dp = sh_make_div(pr), dc = sh_make_div(cols);
+#define SH_EWA(OP, U, F) hipLaunchKernelGGL((k_elementwise_any<OP, U, F>), grid, block, 0, st, Y, A, B, cols, dp, dc, (uint64_t)ld, s, items, (uint32_t)total)
+#define SH_EWA2(OP) do { if (flat) { if (one) SH_EWA(OP, 1, true); else SH_EWA(OP, 4, true); } \
+                         else { if (one) SH_EWA(OP, 1, false); else SH_EWA(OP, 4, false); } } while (0)
+            switch (op) {
+                case OP_GELU: if (flat) SH_EWA(OP_GELU, 1, true); else SH_EWA(OP_GELU, 1, false); break;
+                case OP_ADD: SH_EWA2(OP_ADD); break;
+                case OP_BIAS: SH_EWA2(OP_BIAS); break;
+                case OP_SILU_MUL: SH_EWA2(OP_SILU_MUL); break;
+                default: SH_EWA2(OP_SCALE); break;
+            }
+#undef SH_EWA2
+#undef SH_EWA
+            sh_launch_ok(name);
+            return;
+        }
+    }
     const bool vec = vec_ok(cols, {y, a, b}, {ld});
     const uint32_t per_row = vec ? cols / 8 : cols;
     const uint64_t items64 = (uint64_t)rows * per_row;
@@ -674,7 +799,7 @@ constexpr uint32_t kLlmPad = 0xFFFFu;      // SH_LLM_PAD
 __device__ __forceinline__ uint32_t comp4r(const uint4 &q, int i) { return i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w; }
 
 // y = x rsqrt(mean(x^2) + eps) gamma per row, fp32 statistics (sh_llm.inc.c:91-120). Same layout as k_layernorm.
-template <int NCH, bool VEC>
+template <int NCH, int VEC>
 __global__ __launch_bounds__(256) void k_rmsnorm(uint16_t *y, const uint16_t *x, const uint16_t *gamma, uint32_t rows,
                                                  uint32_t cols, uint64_t ld, float eps) {
     const int lane = threadIdx.x & 63;
@@ -683,10 +808,12 @@ __global__ __launch_bounds__(256) void k_rmsnorm(uint16_t *y, const uint16_t *x,
     float v[NCH][8], g[NCH][8];
     if (VEC) {
         uint4 rx[NCH], rg[NCH];
-        load_raw<NCH>(x + row * ld, cols, lane, rx);
-        load_raw<NCH>(gamma, cols, lane, rg);
+        load_raw<NCH, VEC>(x + row * ld, cols, lane, rx);
+        load_raw<NCH, VEC>(gamma, cols, lane, rg);
 #pragma unroll
         for (int u = 0; u < NCH; ++u) { pin4(rx[u]); pin4(rg[u]); }
+        place_raw<NCH, VEC>(rx, cols, lane);
+        place_raw<NCH, VEC>(rg, cols, lane);
         unpack_row<NCH>(rx, cols, lane, v);
         unpack_row<NCH>(rg, cols, lane, g);
     } else {
@@ -708,7 +835,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm(uint16_t *y, const uint16_t *x,
 
 // softmax(scale x) per row over the keys j with tok_k[j] <= tok_q[row] (unsigned); a padding query row, or one
 // with no allowed key, is uniform 1/cols (sh_llm.inc.c:175-248; run.py:186-196). c = scale log2(e) > 0.
-template <int NCH, bool VEC>
+template <int NCH, int VEC>
 __global__ __launch_bounds__(256) void k_softmax_masked(uint16_t *y, const uint16_t *x, uint32_t rows, uint32_t cols, uint64_t ld,
                                                         float c, const uint16_t *tok_q, const uint16_t *tok_k) {
     const int lane = threadIdx.x & 63;
@@ -721,15 +848,15 @@ __global__ __launch_bounds__(256) void k_softmax_masked(uint16_t *y, const uint1
 #pragma unroll
     for (int u = 0; u < NCH; ++u) {
         if (VEC) {
-            const uint32_t c0 = slot_col<true>(lane, u, 0);
-            const uint4 t = *(const uint4 *)(tok_k + (c0 < cols ? c0 : 0u));
+            const uint32_t c0 = slot_col<VEC>(lane, u, 0);
+            const uint4 t = VEC == ANY ? sh_ld8_row(tok_k, c0 < cols ? c0 : 0u, cols) : *(const uint4 *)(tok_k + (c0 < cols ? c0 : 0u));
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 keep[u][i] = c0 + i < cols && ((comp4r(t, i >> 1) >> (16 * (i & 1))) & 0xFFFFu) <= ti;
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const uint32_t col = slot_col<false>(lane, u, i);
+                const uint32_t col = slot_col<SCALAR>(lane, u, i);
                 keep[u][i] = col < cols && (uint32_t)tok_k[col] <= ti;
             }
         }
@@ -910,8 +1037,9 @@ void sh_softmax_rows(uint64_t y, uint64_t x, uint32_t rows, uint32_t cols, uint3
         return;
     }
     const dim3 grid(sh_cdiv(rows, kRowWaves)), block(256);
-#define SH_SM(N) do { if (vec) hipLaunchKernelGGL((k_softmax<N, true>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c); \
-                      else hipLaunchKernelGGL((k_softmax<N, false>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c); } while (0)
+#define SH_SM(N) do { if (vec) hipLaunchKernelGGL((k_softmax<N, ALIGNED>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c); \
+                      else if (cols >= 8) hipLaunchKernelGGL((k_softmax<N, ANY>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c); \
+                      else hipLaunchKernelGGL((k_softmax<1, SCALAR>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c); } while (0)
     if (cols <= 512) SH_SM(1); else if (cols <= 1024) SH_SM(2); else if (cols <= 2048) SH_SM(4); else if (cols <= 4096) SH_SM(8); else SH_SM(16);
 #undef SH_SM
     sh_launch_ok("sh_softmax_rows");
@@ -951,6 +1079,9 @@ void sh_transpose(uint64_t dst, uint64_t src, uint32_t rows, uint32_t cols, uint
             hipLaunchKernelGGL((k_transpose8<true>), grid, dim3(256), 0, st, D, S, rows, cols, (uint64_t)ld_src, (uint64_t)ld_dst);
         else
             hipLaunchKernelGGL((k_transpose8<false>), grid, dim3(256), 0, st, D, S, rows, cols, (uint64_t)ld_src, (uint64_t)ld_dst);
+    } else if (cols >= 8 && rows >= 8) {
+        hipLaunchKernelGGL((k_transpose8<false, true>), dim3(sh_cdiv(cols, 128), sh_cdiv(rows, 128)), dim3(256), 0, st, D, S, rows, cols,
+                           (uint64_t)ld_src, (uint64_t)ld_dst);
     } else {
         const dim3 grid(sh_cdiv(cols, 32), sh_cdiv(rows, 32));
         hipLaunchKernelGGL(k_transpose1, grid, dim3(256), 0, st, D, S, rows, cols, (uint64_t)ld_src, (uint64_t)ld_dst);
@@ -969,8 +1100,9 @@ void sh_rmsnorm(uint64_t y, uint64_t x, uint64_t gamma, uint32_t rows, uint32_t 
     const dim3 grid(sh_cdiv(rows, kRowWaves)), block(256);
     const bool vec = vec_ok(cols, {y, x, gamma}, {ld});
     uint16_t *Y = (uint16_t *)y; const uint16_t *X = (const uint16_t *)x, *G = (const uint16_t *)gamma;
-#define SH_RMS(N) do { if (vec) hipLaunchKernelGGL((k_rmsnorm<N, true>), grid, block, 0, st, Y, X, G, rows, cols, (uint64_t)ld, eps); \
-                       else hipLaunchKernelGGL((k_rmsnorm<N, false>), grid, block, 0, st, Y, X, G, rows, cols, (uint64_t)ld, eps); } while (0)
+#define SH_RMS(N) do { if (vec) hipLaunchKernelGGL((k_rmsnorm<N, ALIGNED>), grid, block, 0, st, Y, X, G, rows, cols, (uint64_t)ld, eps); \
+                       else if (cols >= 8) hipLaunchKernelGGL((k_rmsnorm<N, ANY>), grid, block, 0, st, Y, X, G, rows, cols, (uint64_t)ld, eps); \
+                      else hipLaunchKernelGGL((k_rmsnorm<1, SCALAR>), grid, block, 0, st, Y, X, G, rows, cols, (uint64_t)ld, eps); } while (0)
     if (cols <= 512) SH_RMS(1); else if (cols <= 1024) SH_RMS(2); else if (cols <= 2048) SH_RMS(4); else if (cols <= 4096) SH_RMS(8); else SH_RMS(16);
 #undef SH_RMS
     sh_launch_ok("sh_rmsnorm");
@@ -1013,8 +1145,9 @@ void sh_softmax_masked(uint64_t y, uint64_t x, uint32_t rows, uint32_t cols, uin
     const dim3 grid(sh_cdiv(rows, kRowWaves)), block(256);
     const bool vec = vec_ok(cols, {y, x, tok_k}, {ld});
     uint16_t *Y = (uint16_t *)y; const uint16_t *X = (const uint16_t *)x, *TQ = (const uint16_t *)tok_q, *TK = (const uint16_t *)tok_k;
-#define SH_SMM(N) do { if (vec) hipLaunchKernelGGL((k_softmax_masked<N, true>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c, TQ, TK); \
-                       else hipLaunchKernelGGL((k_softmax_masked<N, false>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c, TQ, TK); } while (0)
+#define SH_SMM(N) do { if (vec) hipLaunchKernelGGL((k_softmax_masked<N, ALIGNED>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c, TQ, TK); \
+                       else if (cols >= 8) hipLaunchKernelGGL((k_softmax_masked<N, ANY>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c, TQ, TK); \
+                      else hipLaunchKernelGGL((k_softmax_masked<1, SCALAR>), grid, block, 0, st, Y, X, rows, cols, (uint64_t)ld, c, TQ, TK); } while (0)
     if (cols <= 512) SH_SMM(1); else if (cols <= 1024) SH_SMM(2); else if (cols <= 2048) SH_SMM(4); else if (cols <= 4096) SH_SMM(8); else SH_SMM(16);
 #undef SH_SMM
     sh_launch_ok("sh_softmax_masked");
