@@ -439,6 +439,63 @@ __global__ __launch_bounds__(256) void k_softmax_narrow(uint16_t *y, const uint1
     }
 }
 
+// Rows of 257 to 4096 columns (16-byte aligned): as k_layernorm_p, rows spread over LPR-lane groups that walk the rows with
+// the next row's loads in flight, so a wavefront never waits for one row's memory latency between its reductions. Same
+// arithmetic as k_softmax, which keeps few rows. One row per wavefront against this, us: [32768 x 768] 25.0 / 22.2 (a copy of
+// those bytes 21.0), [131072 x 768] 81.1 / 62.2 (60.7), [65536 x 384] 27.4 / 20.7, [12288 x 512] 8.2 / 6.9, [8192 x 3072] 24.3 / 23.1.
+template <int LPR, int NCH, bool NT>
+__global__ __launch_bounds__(256) void k_softmax_p(uint16_t *y, const uint16_t *x, uint32_t rows, uint32_t cols, uint64_t ld, float c) {
+    constexpr int GPW = 64 / LPR;
+    const int lane = threadIdx.x & 63, gl = lane % LPR;
+    const uint32_t group = (blockIdx.x * 4 + (threadIdx.x >> 6)) * GPW + lane / LPR;
+    const uint32_t ngroups = gridDim.x * 4 * GPW;
+    auto col = [&](int u) { return 8u * (uint32_t)(gl + LPR * u); };
+    uint32_t row = group;
+    uint4 cur[NCH];
+    const uint32_t r0 = row < rows ? row : 0u;
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) cur[u] = ld16<false>(x + r0 * ld + (col(u) < cols ? col(u) : 0u));
+    for (; row < rows; row += ngroups) {                  // (in place: a row is read by its own group only, before its stores)
+        const uint32_t nrow = row + ngroups < rows ? row + ngroups : row;
+        float v[NCH][8];
+        float m = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) {
+            unpack8(cur[u], v[u]);
+            const bool ok = col(u) < cols;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                v[u][i] *= c;
+                if (ok) m = fmaxf(m, v[u][i]);
+            }
+        }
+        uint4 nxt[NCH];
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) nxt[u] = ld16<false>(x + nrow * ld + (col(u) < cols ? col(u) : 0u));
+        m = group_max<LPR, 1>(m);
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) {
+            const bool ok = col(u) < cols;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                v[u][i] = ok ? sh_fast_exp2(v[u][i] - m) : 0.f;
+                s += v[u][i];
+            }
+        }
+        const float inv = 1.f / group_sum<LPR, 1>(s);
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) {
+            if (col(u) >= cols) continue;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[u][i] *= inv;
+            st16(y + row * ld + col(u), pack8(v[u]), NT);
+        }
+#pragma unroll
+        for (int u = 0; u < NCH; ++u) cur[u] = nxt[u];
+    }
+}
+
 // Rows wider than the register-resident kernels hold: one 256-thread block per row, three passes over it.
 __device__ float block_reduce(float v, bool is_max, float *red) {
     v = is_max ? sh_wave_max(v) : sh_wave_sum(v);
@@ -1033,6 +1090,19 @@ void sh_softmax_rows(uint64_t y, uint64_t x, uint32_t rows, uint32_t cols, uint3
         if (lpr == 8) { if (nt) hipLaunchKernelGGL((k_softmax_narrow<8, RIT, true>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); else hipLaunchKernelGGL((k_softmax_narrow<8, RIT, false>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); }
         else if (lpr == 16) { if (nt) hipLaunchKernelGGL((k_softmax_narrow<16, RIT, true>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); else hipLaunchKernelGGL((k_softmax_narrow<16, RIT, false>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); }
         else { if (nt) hipLaunchKernelGGL((k_softmax_narrow<32, RIT, true>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); else hipLaunchKernelGGL((k_softmax_narrow<32, RIT, false>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); }
+        sh_launch_ok("sh_softmax_rows");
+        return;
+    }
+    if (vec && cols <= 4096 && rows >= 2048) {      // (fewer rows: one per wavefront, more workgroups: [256 x 768] 3.0 against 3.1)
+        const uint32_t lpr = cols <= 1024 ? 32 : 64, gpb = 4 * (64 / lpr);
+        const uint32_t cap = (uint32_t)(sh_num_cus() > 0 ? sh_num_cus() : 256) * 32;
+        const dim3 g(std::max<uint32_t>(1, std::min<uint32_t>(sh_cdiv(rows, gpb), cap)));
+        const bool nt = (uint64_t)rows * cols * 2 >= kNtBytes;
+#define SH_SMP(L, N) do { if (nt) hipLaunchKernelGGL((k_softmax_p<L, N, true>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); \
+                         else hipLaunchKernelGGL((k_softmax_p<L, N, false>), g, dim3(256), 0, st, Y, X, rows, cols, (uint64_t)ld, c); } while (0)
+        if (lpr == 32) { if (cols <= 512) SH_SMP(32, 2); else if (cols <= 768) SH_SMP(32, 3); else SH_SMP(32, 4); }
+        else { if (cols <= 2048) SH_SMP(64, 4); else if (cols <= 3072) SH_SMP(64, 6); else SH_SMP(64, 8); }
+#undef SH_SMP
         sh_launch_ok("sh_softmax_rows");
         return;
     }
