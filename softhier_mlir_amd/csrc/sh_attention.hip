@@ -1107,7 +1107,8 @@ __global__ __launch_bounds__(256) void k_attn_rows(AttnArgs a) {
 // stamps: device buffer of 8 s_memrealtime values written by the last stamped launch (see attn_stamp)
 struct AttnProfile {
     hipEvent_t e0 = nullptr, e1 = nullptr; bool valid = false; uint32_t entry_ns = 0;
-    uint64_t *stamps = nullptr; bool stamped = false;       // stamped: the last launch's kernel wrote the stamps
+    uint64_t *stamps = nullptr; bool stamped = false;       // stamped: the last launch's kernel wrote the stamps ...
+    hipStream_t stream = nullptr;                           // ... on this stream
 };
 AttnProfile g_prof;
 
@@ -1177,12 +1178,13 @@ int run(uint64_t q, uint64_t k, uint64_t v, uint64_t o, uint32_t B, uint32_t S, 
         if (!events) hipLaunchKernelGGL(kern, grid, dim3(256), (uint32_t)shm, st, a);
         else hipExtLaunchKernelGGL(kern, grid, dim3(256), (uint32_t)shm, st, g_prof.e0, g_prof.e1, 0u, a);
     };
-    // kernels that also write the phase stamps of their last workgroup (only on a stamped, uncaptured call)
+    // Kernels that write the phase stamps of their last workgroup themselves (on a stamped, uncaptured call) need no events:
+    // a dispatch that carries them costs the host 6 us more (9.8 against 3.8) and holds up the kernel behind it.
     uint64_t *sp = events ? g_prof.stamps : nullptr;
+    g_prof.stream = st;
     auto go2 = [&](auto kern, dim3 grid, size_t shm) {
         g_prof.stamped = sp != nullptr;
-        if (!events) hipLaunchKernelGGL(kern, grid, dim3(256), (uint32_t)shm, st, a, sp);
-        else hipExtLaunchKernelGGL(kern, grid, dim3(256), (uint32_t)shm, st, g_prof.e0, g_prof.e1, 0u, a, sp);
+        hipLaunchKernelGGL(kern, grid, dim3(256), (uint32_t)shm, st, a, sp);
     };
     const bool vec = dh % 8 == 0 && ldq % 8 == 0 && ldk % 8 == 0 && ldv % 8 == 0 && ldo % 8 == 0 &&
                      bsq % 8 == 0 && bsk % 8 == 0 && bsv % 8 == 0 && bso % 8 == 0 &&
@@ -1220,8 +1222,7 @@ int run(uint64_t q, uint64_t k, uint64_t v, uint64_t o, uint32_t B, uint32_t S, 
         const dim3 gr((uint32_t)items + pfb), bl(64 * waves);
         const ShDiv dx = sh_make_div(sh_cdiv(S, 32)), dhd = sh_make_div(H);
         g_prof.stamped = sp != nullptr;
-        if (!events) hipLaunchKernelGGL(sfn, gr, bl, lds, st, a, dx, dhd, (uint32_t)items, sp);
-        else hipExtLaunchKernelGGL(sfn, gr, bl, lds, st, g_prof.e0, g_prof.e1, 0u, a, dx, dhd, (uint32_t)items, sp);
+        hipLaunchKernelGGL(sfn, gr, bl, lds, st, a, dx, dhd, (uint32_t)items, sp);
         a.pfl0 = a.pfl1 = 0;
     } else if (tok) {
         if (S > 16384) { sh_set_error(-1, "[sh_attention] masked heads with dh=%u support S <= 16384", dh); return -1; }
@@ -1379,12 +1380,15 @@ int sh_attention_gqa(uint64_t q, uint64_t k, uint64_t v, uint64_t o, uint32_t S,
 uint32_t sh_attention_profile(uint32_t, uint32_t, uint32_t phase) {
     if (!g_prof.valid) return 0;
     phase &= 7;
-    if (hipEventSynchronize(g_prof.e1) != hipSuccess) return 0;
-    uint64_t st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (g_prof.stamped && hipMemcpy(st, g_prof.stamps, sizeof st, hipMemcpyDeviceToHost) == hipSuccess && st[7] && st[6] >= st[7]) {
+    if (g_prof.stamped) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(g_prof.stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
+            hipStreamSynchronize(g_prof.stream) != hipSuccess) { (void)hipGetLastError(); return 0; }
+        uint64_t st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (hipMemcpy(st, g_prof.stamps, sizeof st, hipMemcpyDeviceToHost) != hipSuccess || !st[7] || st[6] < st[7]) return 0;
         return phase == 7 ? 0u : (uint32_t)((st[phase] >= st[7] ? st[phase] - st[7] : 0) * 10u);   // 100 MHz counter
     }
-    if (phase != 6) return 0;
+    if (phase != 6 || hipEventSynchronize(g_prof.e1) != hipSuccess) return 0;
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, g_prof.e0, g_prof.e1) != hipSuccess) return 0;
     return (uint32_t)((double)ms * 1e6 + 0.5);
