@@ -1107,8 +1107,7 @@ __global__ __launch_bounds__(256) void k_attn_rows(AttnArgs a) {
 // stamps: device buffer of 8 s_memrealtime values written by the last stamped launch (see attn_stamp)
 struct AttnProfile {
     hipEvent_t e0 = nullptr, e1 = nullptr; bool valid = false; uint32_t entry_ns = 0;
-    uint64_t *stamps = nullptr; bool stamped = false;       // stamped: the last launch's kernel wrote the stamps ...
-    hipStream_t stream = nullptr;                           // ... on this stream
+    uint64_t *stamps = nullptr; bool stamped = false;       // stamped: the last launch's kernel wrote the stamps
 };
 AttnProfile g_prof;
 
@@ -1181,7 +1180,6 @@ int run(uint64_t q, uint64_t k, uint64_t v, uint64_t o, uint32_t B, uint32_t S, 
     // Kernels that write the phase stamps of their last workgroup themselves (on a stamped, uncaptured call) need no events:
     // a dispatch that carries them costs the host 6 us more (9.8 against 3.8) and holds up the kernel behind it.
     uint64_t *sp = events ? g_prof.stamps : nullptr;
-    g_prof.stream = st;
     auto go2 = [&](auto kern, dim3 grid, size_t shm) {
         g_prof.stamped = sp != nullptr;
         hipLaunchKernelGGL(kern, grid, dim3(256), (uint32_t)shm, st, a, sp);
@@ -1207,8 +1205,7 @@ int run(uint64_t q, uint64_t k, uint64_t v, uint64_t o, uint32_t B, uint32_t S, 
             default: return nullptr;
         }
     };
-    static const int split_max = [] { const char *e = getenv("SH_ATTN_SPLIT"); return (e && *e) ? atoi(e) : -1; }();
-    const uint64_t items = (uint64_t)sh_cdiv(S, 32) * H * B, simds = split_max >= 0 ? (uint64_t)split_max : 4 * (uint64_t)(sh_num_cus() > 0 ? sh_num_cus() : 256);
+    const uint64_t items = (uint64_t)sh_cdiv(S, 32) * H * B, simds = 4 * (uint64_t)(sh_num_cus() > 0 ? sh_num_cus() : 256);
     const uint32_t waves = std::min<uint32_t>(sh_cdiv(S, KB), dh > 64 ? 4 : 8);
     const auto sfn = vec && (tok || (impl == 0 && waves > 2 && items * waves <= simds)) && items < (1u << 30) ? split_fn() : nullptr;
     if (sfn) {
@@ -1382,8 +1379,8 @@ uint32_t sh_attention_profile(uint32_t, uint32_t, uint32_t phase) {
     phase &= 7;
     if (g_prof.stamped) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(g_prof.stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
-            hipStreamSynchronize(g_prof.stream) != hipSuccess) { (void)hipGetLastError(); return 0; }
+        if (hipStreamIsCapturing(sh_stream(), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
+            hipDeviceSynchronize() != hipSuccess) { (void)hipGetLastError(); return 0; }     // (the call's stream may be gone by now)
         uint64_t st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         if (hipMemcpy(st, g_prof.stamps, sizeof st, hipMemcpyDeviceToHost) != hipSuccess || !st[7] || st[6] < st[7]) return 0;
         return phase == 7 ? 0u : (uint32_t)((st[phase] >= st[7] ? st[phase] - st[7] : 0) * 10u);   // 100 MHz counter

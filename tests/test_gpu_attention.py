@@ -149,6 +149,25 @@ def test_profile_reports_the_kernel_time(lib, gpu):
     assert lib.sh_attention_profile(S, 64, 6) > lib.sh_attention_profile(S, 64, 7) == 0
 
 
+def test_profile_after_the_stream_of_the_call_is_gone(lib, gpu):
+    """The stamps are read after the call's work is done, also when its stream was destroyed or another took its place
+    (the HIP calls resolve through the library's own dependency)."""
+    import ctypes
+    S, D, H = 256, 768, 12
+    q = to_dev(data.normal((S, D), 1))
+    O = _zeros(S, D)
+    lib.sh_barrier_global()
+    prev, h = lib.sh_get_stream(), ctypes.c_void_p()
+    assert lib.hipStreamCreate(ctypes.byref(h)) == 0
+    lib.sh_set_stream(h.value)
+    try:
+        assert lib.sh_attention(A(q), A(q), A(q), A(O), S, D, H, D, D, D, D, 0.125, ALL) == 0
+    finally:
+        lib.sh_set_stream(prev)
+        assert lib.hipStreamDestroy(h) == 0
+    assert lib.sh_attention_profile(S, 64, 6) > 0
+
+
 @pytest.mark.parametrize("S", [256, 1024])
 def test_profile_phase_stamps_are_monotone(lib, gpu, S):
     """sh_attention_profile (reference sh_attention.inc.c:67-76, sh_ops.h:124-127): the last workgroup's stamps in
