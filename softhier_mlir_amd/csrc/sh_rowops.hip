@@ -235,8 +235,7 @@ __global__ __launch_bounds__(256) void k_layernorm_p(uint16_t *y, const uint16_t
 #pragma unroll
             for (int i = 0; i < 8; ++i) { v[u][i] = ok ? v[u][i] : 0.f; s += v[u][i]; }
         }
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        s = sh_wave_sum<LPR>(s);
         const float mean = s * inv_n;
         float q = 0.f;
 #pragma unroll
@@ -245,8 +244,7 @@ __global__ __launch_bounds__(256) void k_layernorm_p(uint16_t *y, const uint16_t
 #pragma unroll
             for (int i = 0; i < 8; ++i) { const float d = ok ? v[u][i] - mean : 0.f; q += d * d; }
         }
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
+        q = sh_wave_sum<LPR>(q);
         const float rs = sh_fast_rsq(q * inv_n + eps);
 #pragma unroll
         for (int u = 0; u < NCH; ++u) {
@@ -290,8 +288,7 @@ __global__ __launch_bounds__(256) void k_row_stats(float2 *stats, const uint16_t
 #pragma unroll
             for (int i = 0; i < 8; ++i) { v[u][i] = ok ? v[u][i] : 0.f; s += v[u][i]; }
         }
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        s = sh_wave_sum<LPR>(s);
         const float mean = s * inv_n;
         float q = 0.f;
 #pragma unroll
@@ -300,8 +297,7 @@ __global__ __launch_bounds__(256) void k_row_stats(float2 *stats, const uint16_t
 #pragma unroll
             for (int i = 0; i < 8; ++i) { const float d = ok ? v[u][i] - mean : 0.f; q += d * d; }
         }
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
+        q = sh_wave_sum<LPR>(q);
         if (gl == 0) stats[row] = make_float2(mean, sh_fast_rsq(q * inv_n + eps));
 #pragma unroll
         for (int u = 0; u < NCH; ++u) cur[u] = nxt[u];
@@ -386,19 +382,6 @@ __global__ __launch_bounds__(256) void k_softmax(uint16_t *y, const uint16_t *x,
 // Short rows (cols <= 8 LPR, 16-byte aligned): LPR lanes per row, 64 / LPR rows per wavefront and RIT such
 // groups per wavefront, every load of the RIT groups issued before the first reduction, so each lane keeps RIT
 // 16-byte loads in flight and no lane idles on a row narrower than a wavefront. Same arithmetic as k_softmax.
-template <int LPR, int RIT>
-__device__ __forceinline__ float group_max(float v) {
-#pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-template <int LPR, int RIT>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
 template <int LPR, int RIT, bool NT>
 __global__ __launch_bounds__(256) void k_softmax_narrow(uint16_t *y, const uint16_t *x, uint32_t rows, uint32_t cols, uint64_t ld, float c) {
     constexpr int RPW = 64 / LPR;                     // rows per wavefront per group
@@ -424,14 +407,14 @@ __global__ __launch_bounds__(256) void k_softmax_narrow(uint16_t *y, const uint1
             v[i] *= c;
             if (colok) m = fmaxf(m, v[i]);
         }
-        m = group_max<LPR, RIT>(m);
+        m = sh_wave_max<LPR>(m);
         float sum = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             v[i] = colok ? sh_fast_exp2(v[i] - m) : 0.f;
             sum += v[i];
         }
-        const float inv = 1.f / group_sum<LPR, RIT>(sum);
+        const float inv = 1.f / sh_wave_sum<LPR>(sum);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] *= inv;
         const uint32_t row = row0 + (uint32_t)(r * RPW);
@@ -472,7 +455,7 @@ __global__ __launch_bounds__(256) void k_softmax_p(uint16_t *y, const uint16_t *
         uint4 nxt[NCH];
 #pragma unroll
         for (int u = 0; u < NCH; ++u) nxt[u] = ld16<false>(x + nrow * ld + (col(u) < cols ? col(u) : 0u));
-        m = group_max<LPR, 1>(m);
+        m = sh_wave_max<LPR>(m);
         float s = 0.f;
 #pragma unroll
         for (int u = 0; u < NCH; ++u) {
@@ -483,7 +466,7 @@ __global__ __launch_bounds__(256) void k_softmax_p(uint16_t *y, const uint16_t *
                 s += v[u][i];
             }
         }
-        const float inv = 1.f / group_sum<LPR, 1>(s);
+        const float inv = 1.f / sh_wave_sum<LPR>(s);
 #pragma unroll
         for (int u = 0; u < NCH; ++u) {
             if (col(u) >= cols) continue;
