@@ -177,6 +177,14 @@ __device__ __forceinline__ uint4 sh_fix8(uint4 v, uint32_t sh, uint32_t nv) {
     hi &= mh;
     return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
 }
+// v shifted up by k halves, zeros below (1 <= k <= 7).
+__device__ __forceinline__ uint4 sh_up8(uint4 v, uint32_t k) {
+    uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
+    if (k & 4u) { hi = lo; lo = 0; }
+    const uint32_t s = (k & 3u) * 16u;
+    if (s) { hi = (hi << s) | (lo >> (64u - s)); lo <<= s; }
+    return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
 // Halves [c, c + 8) of a row of n >= 8 halves (zeros past its end; nothing past it is read): a chunk that reaches past the
 // end is loaded from the row's last 8 halves and shifted. c < n.
 __device__ __forceinline__ uint4 sh_ld8_row(const uint16_t *row, uint32_t c, uint32_t n) {
