@@ -177,6 +177,14 @@ __device__ __forceinline__ uint4 sh_fix8(uint4 v, uint32_t sh, uint32_t nv) {
     hi &= mh;
     return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
 }
+// v shifted down by k halves, zeros above (1 <= k <= 7).
+__device__ __forceinline__ uint4 sh_down8(uint4 v, uint32_t k) {
+    uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
+    if (k & 4u) { lo = hi; hi = 0; }
+    const uint32_t s = (k & 3u) * 16u;
+    if (s) { lo = (lo >> s) | (hi << (64u - s)); hi >>= s; }
+    return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
 // v shifted up by k halves, zeros below (1 <= k <= 7).
 __device__ __forceinline__ uint4 sh_up8(uint4 v, uint32_t k) {
     uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
