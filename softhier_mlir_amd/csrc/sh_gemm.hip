@@ -1641,7 +1641,11 @@ float *scratch_ptr() {
 //  - up to two 64 x 64 tiles per CU: that tile (fold 588 x 2304 x 768: 9.6 against 12.9; 1024 x 2304 (576 tiles): level),
 //    with two K ranges from K = 1024 on while it is at most one per CU (1024 x 768 x 3072 with stats: 13.4 against 15.9
 //    with one range and 27.4 for the table).
-//  - operands without 16-byte alignment, and W^T with K % 64 != 0: never the table, whose element-wise kernels are 4 to
+//  - 16-byte operands whose K is no multiple of 64 would need the any-alignment build, of which one or two K ranges lose to
+//    the table's last-slice and W^T kernels: the table below K = 512 (64 x 512 x 136 3.9 against 4.6, x 456 level, 50 x 720 x 720
+//    6.3 against 5.5), for W^T below 384 (512 x 768 x 136 4.3 against 6.7, 2000 x 1000 x 72 4.9 against 5.8, 64 x 512 x 392 5.9
+//    against 5.3) and up to two 64 x 64 tiles per CU (4096 x 768 x 328 12.0 against 11.0).
+//  - operands without 16-byte alignment, and other W^T with K % 64 != 0: never the table, whose element-wise kernels are 4 to
 //    10 times slower (4096 x 768 x 588: 13 against 83; 1000 x 777 x 588: 8 against 54).
 struct SmallPlan { int tile; uint32_t ranges, kps; };
 SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats, bool ln_reg) {
@@ -1676,6 +1680,7 @@ SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats,
         if (force == SMALL_DMA2 && fast && !r.wt && r.K % 128 == 0) return {force, 1, r.K / 2};
         return none;
     }
+    if (any && vec && r.K < (r.wt ? 384u : 512u) && t64 <= 2 * cus) return none;
     if (t32 <= cus) {
         const SplitK sk = split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, 4 * t32 <= cus ? 8 : 4)));
         return {SMALL_RANGES_32, sk.splits, sk.kps};
