@@ -516,9 +516,8 @@ __global__ __launch_bounds__(256, DH == 64 ? 3 : 2) void k_flash2(AttnArgs a, ui
     attn_stamp(stamp, last, 6);
 }
 
-// One-pass variant of k_flash2 (the default for aligned dh 64 / 128 heads whose scale folds, |c| <= 1, and of
-// 32 / 72 / 80 / 96-wide heads of any scale, without a token mask; against the padded register-staged k_flash, B = 4, S = 580, 16 heads of 80: 65.3 -> 20.6 us, B = 1,
-// S = 1024, 16 heads of 32: 34.0 -> 12.4): each key block's scores come out of the MFMAs already shifted by the query's reference m (the FOLD
+// One-pass variant of k_flash2 (the default for aligned dh 64 / 128 heads whose scale folds, |c| <= 1, and, as EX builds, of
+// 32 / 72 / 80 / 96-wide heads of any scale, without a token mask): each key block's scores come out of the MFMAs already shifted by the query's reference m (the FOLD
 // bias step: ones x (-m_hi, -m_lo)), so p = 2^acc. m starts at 0 and moves to the first block's maximum when that
 // lies more than kTau (log2 units) from 0; a later block is first tested by its numerators' sum per lane (32 keys,
 // formed for the row sum anyway), and only when that exceeds 32 x 2^kTau is its maximum formed and m moved for the
@@ -529,8 +528,11 @@ __global__ __launch_bounds__(256, DH == 64 ? 3 : 2) void k_flash2(AttnArgs a, ui
 // this drops the maximum pass (its score MFMAs, K fragment reads and K DMAs) and the refill of the ring between the
 // passes. Same LDS ring, fragment prefetch and occupancy as k_flash2.
 constexpr float kTau = 8.f;
-// EX (the widths other than 64 and 128, which a kernel with unscaled queries served before): the queries stay as given and
-// c s - m is one fp32 multiply-add per score instead of the scaled fragments and the bias step, so any scale will do.
+// EX (widths 32 / 72 / 80 / 96): k_flash's arithmetic on this kernel's loads: the queries stay as given, m is the running maximum
+// itself and c s - m one fp32 multiply-add per score, so any scale will do and the bits are k_flash's. Against k_flash, padded
+// to 64 or 128: B = 4, S = 580, 16 heads of 80 64.8 -> 22.6 us, B = 1, S = 1024, 16 heads of 32 33.4 -> 13.3. (m left at 0 while the
+// first maximum was within kTau of it took 20.0 and 12.4 us, but numerators up to 2^8 smaller are lost to fp16 sooner: error against
+// float64 2.93e-4 instead of 2.74e-4 on the first of these, 1.4e-2 for a long tail 17 units below its maximum.)
 template <int DH, int NST, bool PF = false, bool ST = true, bool RAG = true, bool EX = false>
 __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, uint64_t *stamp) {
     constexpr int DC = DH / 8, NS = (DC + 1) / 2, DT = (DH + 31) / 32;
@@ -675,7 +677,7 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
 
     sh_f16v oacc[DT];                                // (set by the first block's P.V MFMAs, which start from zero)
     float lsum = 0.f;                                // this lane's keys' fp16 numerators, summed in fp32
-    float mrun = 0.f;                                // reference m of this lane's query (c s units)
+    float mrun = EX ? -INFINITY : 0.f;               // reference m of this lane's query (c s units)
     bool biased = false;                             // some lane's m left 0 (wave-uniform): the bias step is needed
     const sh_h2 one2 = {(_Float16)1.0f, (_Float16)1.0f};
     // LDS byte address in stage 0 of each lane's V^T fragment j (rows k0 of its lower half; the upper half's rows
@@ -711,16 +713,9 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
                         if (kb * KB + 32 * tt + 8 * (r >> 2) + 4 * g + (r & 3) >= S) sacc[tt][r] = -INFINITY;
             }
         };
-        auto shift_ex = [&]() {                      // (EX: acc = c s - m)
-#pragma unroll
-            for (int tt = 0; tt < (EX ? 2 : 0); ++tt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sacc[tt][r] = fmaf(sacc[tt][r], a.c, -mrun);
-        };
         if (!EX && biased) scores(stc, sacc, Biased{});
         else scores(stc, sacc, std::false_type{});   // (while every m is 0 the bias step would add zeros)
-        shift_ex();
-        mask_tail();
+        if constexpr (!EX) mask_tail();
         // V^T fragment j: substep j / DT, d tile j % DT (consecutive MFMAs alternate accumulators)
         auto vfrag = [&](int j) -> sh_h8 {
             const uint32_t at = vaddr[j] + (uint32_t)st * STAGE;
@@ -729,18 +724,51 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
             return __builtin_bit_cast(sh_h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         };
         sh_h8 pf[4];                                 // numerators p = 2^acc, fp16, as the P.V MFMA operands
-        float pex[4];                                // EX: the sums of the unrounded numerators, as k_flash sums them
         auto expo = [&]() {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) pex[e] = 0.f;
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) pf[2 * tt + (r >> 3)][r & 7] = (_Float16)sh_fast_exp2(sacc[tt][r]);
+        };
+        // EX: k_flash's step, in its order, so it stores k_flash's bits: m is the running maximum of c s (exactly, so the
+        // largest numerator is 1 and none is lost to fp16 that k_flash keeps), l the sum of the unrounded numerators. O and l
+        // are rescaled only when some lane's m moved (else by 1).
+        auto step_ex = [&]() {
+            float e0, e1;                            // (rows past S hold key S - 1's scores: no other extreme)
+            if (a.c >= 0.f) {
+                e0 = e1 = -INFINITY;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { e0 = fmaxf(e0, sacc[0][r]); e1 = fmaxf(e1, sacc[1][r]); }
+                e0 = sh_max_xor32(fmaxf(e0, e1));
+            } else {
+                e0 = e1 = INFINITY;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { e0 = fminf(e0, sacc[0][r]); e1 = fminf(e1, sacc[1][r]); }
+                e0 = -sh_max_xor32(-fminf(e0, e1));
+            }
+            const float mn = fmaxf(mrun, a.c * e0);
+            float alpha = 1.f;
+            if (!first && __ballot(mn != mrun) != 0) {
+                alpha = sh_fast_exp2(mrun - mn);
+#pragma unroll
+                for (int i = 0; i < DT; ++i) oacc[i] *= alpha;
+            }
+            mrun = mn;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sacc[tt][r] = fmaf(sacc[tt][r], a.c, -mn);
+            mask_tail();
+            float ps = 0.f;
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const float p = sh_fast_exp2(sacc[tt][r]);
-                    if constexpr (EX) pex[r & 3] += p;
+                    ps += p;
                     pf[2 * tt + (r >> 3)][r & 7] = (_Float16)p;
                 }
+            lsum = first ? ps : fmaf(lsum, alpha, ps);
         };
         // The first V fragments are read now and the numerators formed before the maximum test (formed again in
         // the rare case that m moves): the exponentials then hide those reads' latency and the maximum's chain,
@@ -749,11 +777,11 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
         sh_h8 vr[VA + 1];
 #pragma unroll
         for (int j = 0; j < VA; ++j) vr[j] = vfrag(j);
-        expo();
+        if constexpr (EX) step_ex();
+        else expo();
         // this lane's sum of the block's fp16 numerators (fp32 sums, four chains): the row sum's share and, for a
         // later block, the test whether m must move
         auto psum = [&]() -> float {
-            if constexpr (EX) return (pex[0] + pex[1]) + (pex[2] + pex[3]);
             float c[4];
 #pragma unroll
             for (int sp = 0; sp < 4; ++sp) {
@@ -778,8 +806,9 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
         // needs anyway: only when some lane's 32 numerators sum past 32 x 2^kTau (so one of them exceeds 2^kTau, and
         // its query's maximum exceeds m by more than kTau) is the maximum formed, and m moves for the queries whose
         // maximum exceeds m by more than kTau, as the first rule would move them.
-        bool test;
-        if constexpr (first) {
+        bool test = false;
+        if constexpr (EX) {
+        } else if constexpr (first) {
             bm = block_max();
             test = __ballot(fabsf(bm) > kTau) != 0;
         } else {
@@ -800,14 +829,9 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
                 lsum *= sc;
             }
             mrun += shift;
-            if constexpr (EX) {
-                scores(stc, sacc, std::false_type{});
-                shift_ex();
-            } else {
-                set_bias(mrun);
-                biased = true;
-                scores(stc, sacc, Biased{});
-            }
+            set_bias(mrun);
+            biased = true;
+            scores(stc, sacc, Biased{});
             mask_tail();
             expo();
             if constexpr (!first) blk = psum();
@@ -815,8 +839,8 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
         if constexpr (first) {
             attn_stamp(stamp, last, 3);
             attn_stamp(stamp, last, 4);
-            lsum = psum();
-        } else {
+            if constexpr (!EX) lsum = psum();
+        } else if constexpr (!EX) {
             lsum += blk;
         }
 #pragma unroll

@@ -80,3 +80,56 @@ def test_split_keys_masked(lib, gpu, S, dh):
         assert lib.sh_attention_gqa(A(Q), A(K), A(V), A(O), S, D, H, Hkv, D, DKV, DKV, D, 0.125, A(T, 1), shops.SH_ALL) == 0, shops.last_error()
         bad, err, _ = refs.close(to_np(O), refs.attention_gqa(q, k, v, H, Hkv, tok))
         assert bad == 0, err
+
+
+@pytest.mark.parametrize("dh", [32, 72, 80, 96])
+@pytest.mark.parametrize("S,scale", [(1, 0.125), (63, -0.3), (64, 2.0), (129, 0.125), (300, 0.0), (580, 0.125)])
+def test_one_pass_widths_store_the_general_kernel_bits(lib, gpu, S, scale, dh):
+    """The same heads one element into their buffers run on the register-staged kernel of any alignment: the same running
+    maximum, numerators and sums in the same order, so the same bits, infinite scores included."""
+    import torch
+    B, H = 2, 3
+    D = H * dh
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(B * S, 3 * D, generator=g, device="cuda").half()
+    x[:, :D] *= 4                                             # scores over a few tens: the maximum moves in later blocks
+    x[S // 2, D:D + 2] = float("inf")                         # one key of head 0, sequence 0: scores +-inf and NaN
+    outs = []
+    for off in (0, 1):
+        xb = torch.zeros(B * S * 3 * D + 8, device="cuda", dtype=torch.float16)
+        xb[off:off + x.numel()] = x.reshape(-1)
+        ob = torch.zeros(B * S * D + 8, device="cuda", dtype=torch.float16)
+        rc = lib.sh_attention_batched(A(xb, off), A(xb, off + D), A(xb, off + 2 * D), A(ob, off), B, S, D, H, 3 * D, 3 * D, 3 * D, D,
+                                      S * 3 * D, S * 3 * D, S * 3 * D, S * D, scale, 0)
+        assert rc == 0, shops.last_error()
+        outs.append(ob[off:off + B * S * D].clone())
+    nan = [torch.isnan(o) for o in outs]
+    assert torch.equal(*nan)
+    assert torch.equal(outs[0].view(torch.int16)[~nan[0]], outs[1].view(torch.int16)[~nan[0]])
+
+
+@pytest.mark.parametrize("dh", [32, 64, 72, 80, 96, 128])
+def test_low_tail(lib, gpu, dh):
+    """One key a few units above a long tail that is far below 0, the reference of an unmoved exponent: the tail's numerators
+    keep the weight that their row sum counts. Against float64 in units of max|v|: numerators and output rounded to fp16 once
+    each (2^-11 + 2^-11), and the tail's S numerators, fp16 subnormals, by at most 2^-25 of the largest each. (64 and 128 wide heads start
+    from m = 0 while the first maximum is within 8 of it, their numerators up to 2^8 smaller: S 2^-17, and their row sums are those
+    of the rounded numerators.)"""
+    import torch
+    S = 2048
+    q = np.zeros((S, dh), np.float16); k = np.zeros((S, dh), np.float16)
+    q[:, 0] = 1.0
+    top, low = (-7.9, -25.5) if dh not in (64, 128) else (-7.9, -20.0)
+    k[:, 0] = low
+    k[7, 0] = top
+    v = np.abs(data.normal((S, dh), 95)).astype(np.float16) + np.float16(1)
+    v[7] = 0
+    scale = float(np.log(2.0))                                # scores in log2 units
+    O = torch.zeros((S, dh), dtype=torch.float16, device="cuda")
+    rc = lib.sh_attention_batched(A(to_dev(q)), A(to_dev(k)), A(to_dev(v)), A(O), 1, S, dh, 1, dh, dh, dh, dh, 0, 0, 0, 0, scale, 0)
+    assert rc == 0, shops.last_error()
+    t = k[:, 0].astype(np.float64)
+    p = 2.0 ** (t - t.max())
+    want = (p / p.sum()) @ v.astype(np.float64)
+    sub = S * (2.0 ** -17 if dh in (64, 128) else 2.0 ** -25)
+    assert np.abs(to_np(O).astype(np.float64) - want).max() <= (2 * 2.0 ** -11 + sub) * v.max(), dh
