@@ -2,6 +2,7 @@
 // LayerNorm fold and the epilogue chain. Not part of the C ABI.
 #pragma once
 #include "sh_common.h"
+#include "sh_ln_pair.h"
 
 constexpr int BK = 64;
 
@@ -85,16 +86,16 @@ __device__ __forceinline__ void ln_pair_load(const GemmArgs &a, uint32_t gm, LnP
         return;
     }
     if (!ln_in_registers(a)) return;
-    const uint32_t n = a.ln_parts / 2, h0 = (n + 1) / 2, up = (threadIdx.x >> 5) & 1;      // float4s: h0 lower, n - h0 upper
-    const float4 *pp = (const float4 *)((const float2 *)a.ln_stats + (uint64_t)gm * a.ln_parts) + up * h0;
+    const uint32_t n = a.ln_parts / 2, up = (threadIdx.x >> 5) & 1;
+    const float4 *pp = (const float4 *)((const float2 *)a.ln_stats + (uint64_t)gm * a.ln_parts);
 #pragma unroll
     for (int h = 0; h < 8; ++h)
-        if ((uint32_t)h < h0) l.q[h] = pp[min((uint32_t)h, n - h0 * up - 1)];               // (n odd: the upper lane's last is unused)
+        if ((uint32_t)h < ln_pair_count(n, 0)) l.q[h] = pp[ln_pair_at(n, up, h)];           // (n odd: the upper lane's last is unused)
 }
 __device__ __forceinline__ float2 ln_pair_form(const GemmArgs &a, uint32_t gm, const LnPair &l) {
     if (a.ln_parts == 0) return make_float2(l.q[0].x, l.q[0].y);
     if (!ln_in_registers(a)) return ln_row(a, gm);
-    const uint32_t n = a.ln_parts / 2, h0 = (n + 1) / 2, up = (threadIdx.x >> 5) & 1, mine = up ? n - h0 : h0;
+    const uint32_t up = (threadIdx.x >> 5) & 1, mine = ln_pair_count(a.ln_parts / 2, up);
     const int lower = (int)(threadIdx.x & 31), upper = lower + 32;
     const float inv_n = 1.f / (32.f * (float)a.ln_parts);
     float s = 0.f, m2 = 0.f;
