@@ -894,6 +894,8 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
 // all in flight together, the next block's issued before the exponentials), V goes through the wavefront's own LDS stage for the transpose
 // reads, and no barrier is crossed before the combine. p = 2^(c s - m) with the scores in fp32, so any scale and sign.
 // MASK: key j is allowed for query i iff tok[j] <= tok[i]; a padding query averages V uniformly over the S keys.
+// Masked heads of 32 / 72 / 80 / 96 (P2) hold each numerator as two fp16 halves of 2^15 p, 22 bits down to 2^-29, and sum them
+// unrounded: the per-query kernel they would take otherwise keeps p in fp32, and one fp16 half loses a tail below 2^-25 of the maximum.
 // Workgroups past the (query block, head, sequence) items read the caller's prefetch ranges (a.pf0, a.pf1).
 typedef uint32_t attn_u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t attn_u4 __attribute__((ext_vector_type(4)));
@@ -963,6 +965,7 @@ __global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a
     for (int s = 0; s < NS; ++s) qf[s] = (DC & 1) && s == NS - 1 && g == 1 ? sh_h8{} : __builtin_bit_cast(sh_h8, qr[s]);
     const bool uni = MASK && tq == kLlmPad;
     const float c = a.c;
+    constexpr bool P2 = MASK && DH != 64 && DH != 128;
     const sh_h2 one2 = {(_Float16)1.0f, (_Float16)1.0f};
     sh_f16v oacc[DT];
 #pragma unroll
@@ -1006,14 +1009,22 @@ __global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a
         mb = sh_max_xor32(mb);
         const float mn = fmaxf(m, mb), ms = mn == -INFINITY ? 0.f : mn, alpha = sh_fast_exp2(m - ms);
         m = mn;
-        sh_h8 pf[4];
+        sh_h8 pf[4], pl[P2 ? 4 : 1];
+        l *= alpha;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) pf[2 * tt + (r >> 3)][r & 7] = (_Float16)sh_fast_exp2(sacc[tt][r] - ms);
-        l *= alpha;
+            for (int r = 0; r < 16; ++r) {
+                const float p = sh_fast_exp2(sacc[tt][r] - ms) * (P2 ? 32768.f : 1.f);
+                const _Float16 hi = (_Float16)p;
+                pf[2 * tt + (r >> 3)][r & 7] = hi;
+                if constexpr (P2) {
+                    pl[2 * tt + (r >> 3)][r & 7] = (_Float16)(p - (float)hi);
+                    l += p;
+                }
+            }
 #pragma unroll
-        for (int sp = 0; sp < 4; ++sp) {
+        for (int sp = 0; sp < (P2 ? 0 : 4); ++sp) {
             const uint4 w = __builtin_bit_cast(uint4, pf[sp]);
             l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.x), one2, l, false);
             l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.y), one2, l, false);
@@ -1033,6 +1044,7 @@ __global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a
                 const sh_s4 lo = sh_ds_read_tr(at), hi = sh_ds_read_tr(at + 8 * (DH * 2));
                 const sh_h8 vf = __builtin_bit_cast(sh_h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
                 oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[sp], oacc[dt], 0, 0, 0);
+                if constexpr (P2) oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[sp], oacc[dt], 0, 0, 0);
             }
         asm volatile("" ::: "memory");
         if (kb == (uint32_t)wave) { attn_stamp(stamp, last, 3); attn_stamp(stamp, last, 4); }

@@ -133,3 +133,25 @@ def test_low_tail(lib, gpu, dh):
     want = (p / p.sum()) @ v.astype(np.float64)
     sub = S * (2.0 ** -17 if dh in (64, 128) else 2.0 ** -25)
     assert np.abs(to_np(O).astype(np.float64) - want).max() <= (2 * 2.0 ** -11 + sub) * v.max(), dh
+
+
+@pytest.mark.parametrize("dh", [32, 72, 80, 96])
+def test_masked_tail_keeps_fp32_weights(lib, gpu, dh):
+    """Masked heads of these widths weigh keys in fp32: a tail 25.5 (log2) below its maximum, which one fp16 numerator cannot
+    hold, carries the whole output here (the largest key's values are 0). Against float64: the output's rounding 2^-11, fp32 exponents (25.5
+    in log2, 2^-24 relative) 2^-19, S sums 2^-24 each and numerators 2^-22, together below 2^-10."""
+    import torch
+    S = 256
+    q = np.zeros((S, dh), np.float16); k = np.zeros((S, dh), np.float16)
+    q[:, 0] = 1.0
+    k[:, 0] = -25.5
+    k[7, 0] = 0.0
+    v = np.full((S, dh), 60000.0, np.float16) - np.abs(data.normal((S, dh), 96)).astype(np.float16) * np.float16(4096)
+    v[7] = 0
+    T = torch.zeros(S, dtype=torch.int16, device="cuda")      # one class: every key allowed
+    O = torch.zeros((S, dh), dtype=torch.float16, device="cuda")
+    rc = lib.sh_attention_gqa(A(to_dev(q)), A(to_dev(k)), A(to_dev(v)), A(O), S, dh, 1, 1, dh, dh, dh, dh, float(np.log(2.0)), A(T), shops.SH_ALL)
+    assert rc == 0, shops.last_error()
+    p = 2.0 ** k[:, 0].astype(np.float64)
+    want = (p / p.sum()) @ v.astype(np.float64)
+    assert np.abs(to_np(O).astype(np.float64) / want - 1).max() <= 2.0 ** -10
