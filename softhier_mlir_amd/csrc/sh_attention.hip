@@ -893,7 +893,8 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
 // Latency bounds it: K fragments come straight from global memory into registers (each block's K, V and token loads are
 // all in flight together, the next block's issued before the exponentials), V goes through the wavefront's own LDS stage for the transpose
 // reads, and no barrier is crossed before the combine. p = 2^(c s - m) with the scores in fp32, so any scale and sign.
-// MASK: key j is allowed for query i iff tok[j] <= tok[i]; a padding query averages V uniformly over the S keys.
+// MASK: key j is allowed for query i iff tok[j] <= tok[i]; a padding query, or one whose allowed keys all score -inf, averages
+// V uniformly over the S keys.
 // Masked heads of 32 / 72 / 80 / 96 (P2) hold each numerator as two fp16 halves of 2^15 p, 22 bits down to 2^-29, and sum them
 // unrounded: the per-query kernel they would take otherwise keeps p in fp32, and one fp16 half loses a tail below 2^-25 of the maximum.
 // Workgroups past the (query block, head, sequence) items read the caller's prefetch ranges (a.pf0, a.pf1).
@@ -1078,6 +1079,16 @@ __global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a
             lt = fmaf(f, p[32 * OP + 32 + q], lt);
             o[0] = fmaf(f, lo.x, o[0]); o[1] = fmaf(f, lo.y, o[1]); o[2] = fmaf(f, lo.z, o[2]); o[3] = fmaf(f, lo.w, o[3]);
             o[4] = fmaf(f, hi.x, o[4]); o[5] = fmaf(f, hi.y, o[5]); o[6] = fmaf(f, hi.z, o[6]); o[7] = fmaf(f, hi.w, o[7]);
+        }
+        if (MASK && mx == -INFINITY) {               // no key has weight
+            lt = (float)S;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = 0.f;
+            for (uint32_t j = 0; j < S; ++j) {
+                const attn_u4 vv = *(const attn_u4 *)(Vp + (uint64_t)j * a.ldv + 8 * pc);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] += sh_dev_h2f((uint16_t)(vv[e >> 1] >> (16 * (e & 1))));
+            }
         }
         const float inv = 1.f / lt;
         uint32_t w4[4];

@@ -155,3 +155,25 @@ def test_masked_tail_keeps_fp32_weights(lib, gpu, dh):
     p = 2.0 ** k[:, 0].astype(np.float64)
     want = (p / p.sum()) @ v.astype(np.float64)
     assert np.abs(to_np(O).astype(np.float64) / want - 1).max() <= 2.0 ** -10
+
+
+@pytest.mark.parametrize("dh", [32, 64, 72, 80, 96, 128, 88])
+@pytest.mark.parametrize("S", [12, 132])
+def test_masked_infinite_scores(lib, gpu, S, dh):
+    """Keys that score -inf take no weight; a query whose allowed keys all do averages V uniformly over the S keys, as a
+    padding query does. (88 wide heads: the per-query kernel.) Means of values in (0, 4) rounded to fp16 weights and once more."""
+    import torch
+    q, k = np.abs(data.normal((S, dh), 97)) + 1, data.normal((S, dh), 98)
+    v = np.minimum(np.abs(data.normal((S, dh), 99)), 4).astype(np.float16)
+    k[:5, 0] = -np.inf                                        # causal: queries 0 .. 4 see no other key
+    T = torch.arange(S, dtype=torch.int32, device="cuda").to(torch.int16)
+    O = torch.zeros((S, dh), dtype=torch.float16, device="cuda")
+    rc = lib.sh_attention_gqa(A(to_dev(q)), A(to_dev(k)), A(to_dev(v)), A(O), S, dh, 1, 1, dh, dh, dh, dh, 0.125, A(T), shops.SH_ALL)
+    assert rc == 0, shops.last_error()
+    q, k, v = (t.astype(np.float16).astype(np.float64) for t in (q, k, v))
+    want = np.empty((S, dh))
+    for i in range(S):
+        s = 0.125 * (k[5:i + 1] @ q[i])
+        p = np.exp(s - s.max()) if i >= 5 else np.ones(S)
+        want[i] = (p / p.sum()) @ (v[5:i + 1] if i >= 5 else v)
+    assert np.abs(to_np(O).astype(np.float64) - want).max() <= 2 * 2.0 ** -11 * 4 + 2.0 ** -11 * 4
