@@ -232,7 +232,7 @@ int sh_gemm_splitk_noalloc(uint64_t x, uint64_t w, uint64_t z, uint32_t M, uint3
 /* Fused GEMM epilogue: z = act(X.W [+ z_old if cfg->accumulate] + bias) rounded to fp16, then
  * [+ residual, rounded again]. bias: 0 or an fp16 (SH_BIAS_FP16) / fp32 (SH_BIAS_FP32) row of N values.
  * residual: 0 or an fp16 [M,N] tensor with leading dim ldr (may alias z). No tile-divisibility rule and no
- * TCDM budget; M, N, K >= 1. splits: as sh_gemm_splitk (1 = no partials in memory, 0 = library choice). */
+ * TCDM budget; M, N, K >= 1. splits: as sh_gemm_splitk (1 = no split, 0 = library choice). */
 enum { SH_ACT_NONE = 0, SH_ACT_GELU = 1 };
 enum { SH_BIAS_FP16 = 0, SH_BIAS_FP32 = 1 };
 typedef struct {
@@ -271,7 +271,7 @@ int sh_gemm_ex_wt(uint64_t x, uint64_t wt, uint64_t z, uint32_t M, uint32_t N, u
 /* Additive (no counterpart in the reference): the GEMM cost model's plan for an (M, N, K) problem with
  * 16-byte-aligned operands and a split request (0 = library choice): out[0] tile configuration, out[1] /
  * out[2] its tile rows / columns, out[3] the split count. A large problem's first call may still replace the
- * configuration by its one-time timing, and a problem of few tiles without a split request runs on smaller tiles that may
+ * configuration by its one-time timing, and a problem of few tiles runs on smaller tiles instead, which with splits = 0 may
  * sum K in up to eight ranges inside a workgroup (fp32, in range order; deterministic). Runs no GPU work. 0, or -1 for an
  * empty problem / NULL out. */
 int sh_gemm_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t splits, uint32_t *out);

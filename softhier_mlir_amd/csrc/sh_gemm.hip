@@ -1630,23 +1630,28 @@ float *scratch_ptr() {
 }
 
 // Whether a call runs on the small-problem / any-alignment kernels (sh_gemm_small.hip) or the 64 x 64 direct-to-LDS tile
-// with late fold operands, and with how many K ranges per workgroup; tile -1: the tile table. Chosen by sizes and
-// alignment alone, so calls that differ in their epilogue only store the same product bits. The lines were measured on
-// MI355X in replayed graphs (us; fold / stats: with the LayerNorm fold from row partials / bias, residual, row partials):
+// with late fold operands, and with how many K ranges per workgroup; tile -1: the tile table.
+// A call that asks for no split (splits = 1) is one chain of 16-k blocks per output in the direct-to-LDS order whatever kernel it
+// gets here, and the table's for K >= 64, so its bits depend neither on M nor on the epilogue nor (K % 64 == 0, or unaligned) on the
+// weight's layout; the ranges serve calls that leave the split to the library (splits = 0).
+// The lines were measured on MI355X in replayed graphs (us; fold / stats: with the LayerNorm fold from row partials / bias, residual,
+// row partials).
+// One chain:
+//  - up to two 64 x 64 tiles per CU: that tile (256 x 768 x 3072 12.4 against 13.2 for the table, with stats 13.2 against 23.8;
+//    fold 588 x 2304 x 768 8.9 against 11.0; 1024 x 2304 (576 tiles): level).
+//    With the fold on at most one 32 x 32 tile per CU that tile, a wavefront each (256 x 768 x 768 6.3 against 6.8).
+//  - 16-byte operands with K % 64 != 0: W always the table (50 x 2048 x 720 5.8 against 6.7, 256 x 768 x 3080 16.2 against 16.4), W^T
+//    below K = 384 (64 x 512 x 136 3.6 against 4.2, 1000 x 504 x 328 5.1 against 5.4; 50 x 720 x 720 7.3 against 6.5).
+// Ranges:
 //  - up to one 32 x 32 tile per CU: four K ranges of at least 192 k (256 x 768 x 768: 4.5 against 5.2 for the 64 x 64 tile,
-//    fold 5.4 against 11.8, x 3072: 7.3 against 13.0, with stats 8.0 against 23.9; 50 x 720 x 2048: 5.4 against 9.2);
-//    eight where the tiles leave three quarters of the CUs idle. Above one tile per CU they lose (588 x 768: 6.1 against
-//    5.6).
+//    x 3072: 7.3 against 12.4, with stats 8.0 against 13.2); eight where the tiles leave three quarters of the CUs idle. Above one
+//    tile per CU they lose (588 x 768: 6.1 against 5.6).
 //  - up to one 64 x 32 tile per CU with a long K: the same with 64-row tiles.
-//  - up to two 64 x 64 tiles per CU: that tile (fold 588 x 2304 x 768: 9.6 against 12.9; 1024 x 2304 (576 tiles): level),
-//    with two K ranges from K = 1024 on while it is at most one per CU (1024 x 768 x 3072 with stats: 13.4 against 15.9
-//    with one range and 27.4 for the table).
-//  - 16-byte operands whose K is no multiple of 64 would need the any-alignment build, of which one or two K ranges lose to
-//    the table's last-slice and W^T kernels: the table below K = 512 (64 x 512 x 136 3.9 against 4.6, x 456 level, 50 x 720 x 720
-//    6.3 against 5.5), for W^T below 384 (512 x 768 x 136 4.3 against 6.7, 2000 x 1000 x 72 4.9 against 5.8, 64 x 512 x 392 5.9
-//    against 5.3) and up to two 64 x 64 tiles per CU (4096 x 768 x 328 12.0 against 11.0).
-//  - operands without 16-byte alignment, and other W^T with K % 64 != 0: never the table, whose element-wise kernels are 4 to
-//    10 times slower (4096 x 768 x 588: 13 against 83; 1000 x 777 x 588: 8 against 54).
+//  - up to one 64 x 64 tile per CU from K = 1024 on: that tile with two ranges (1024 x 768 x 3072 with stats: 13.4 against 15.9).
+//  - 16-byte operands whose K is no multiple of 64: the table below K = 512 (64 x 512 x 136 3.9 against 4.6, x 456 level), for W^T
+//    below 384, up to two 64 x 64 tiles per CU (4096 x 768 x 328 12.0 against 11.0).
+// Operands without 16-byte alignment, and other W^T with K % 64 != 0: never the table, whose element-wise kernels are 4 to
+// 10 times slower (4096 x 768 x 588: 13 against 83; 1000 x 777 x 588: 8 against 54).
 struct SmallPlan { int tile; uint32_t ranges, kps; };
 SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats, bool ln_reg) {
     const SmallPlan none{-1, 0, 0};
@@ -1672,25 +1677,27 @@ SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats,
         }
     }
     const SplitK one = split_k(r.K, 1);
+    // (one range for a caller that asks for none: splits = 1)
+    auto ranges = [&](uint32_t most) { return r.splits == 0 ? split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, most))) : one; };
     if (force >= 0) {
-        const SplitK sk = split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, 4)));
+        const SplitK sk = ranges(4);
         if (force == SMALL_RANGES_32 || (force == SMALL_RANGES_64 && !ln)) return {force, sk.splits, sk.kps};
         if ((force == SMALL_64x64 || force == SMALL_128x64) && !ln && !stats && r.ldx >= 8 && r.ldw >= 8) return {force, 1, one.kps};
         if (force == SMALL_DMA && fast && !r.wt) return {force, 1, one.kps};
-        if (force == SMALL_DMA2 && fast && !r.wt && r.K % 128 == 0) return {force, 1, r.K / 2};
+        if (force == SMALL_DMA2 && fast && !r.wt && r.K % 128 == 0 && r.splits == 0) return {force, 1, r.K / 2};
         return none;
     }
-    if (any && vec && r.K < (r.wt ? 384u : 512u) && t64 <= 2 * cus) return none;
-    if (t32 <= cus) {
-        const SplitK sk = split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, 4 * t32 <= cus ? 8 : 4)));
+    if (any && vec && t64 <= 2 * cus && (r.wt ? r.K < 384 : r.K < 512 || r.splits != 0)) return none;
+    if (t32 <= cus && (r.splits == 0 || !fast || ln)) {
+        const SplitK sk = ranges(4 * t32 <= cus ? kSmallMaxRanges : kSmallMaxRanges / 2);
         return {SMALL_RANGES_32, sk.splits, sk.kps};
     }
-    if (t64x32 <= cus && !ln && (r.K >= 1024 || !table_ok)) {
-        const SplitK sk = split_k(r.K, std::max<uint32_t>(1, std::min<uint32_t>(r.K / 192, 4)));
+    if (t64x32 <= cus && !ln && r.splits == 0 && (r.K >= 1024 || !table_ok)) {
+        const SplitK sk = ranges(kSmallMaxRanges64);
         return {SMALL_RANGES_64, sk.splits, sk.kps};
     }
     if (fast && !r.wt) {
-        if (t64 <= cus && r.K >= 1024 && r.K % 128 == 0) return {SMALL_DMA2, 1, r.K / 2};
+        if (t64 <= cus && r.K >= 1024 && r.K % 128 == 0 && r.splits == 0) return {SMALL_DMA2, 1, r.K / 2};
         if (t64 <= 2 * cus) return {SMALL_DMA, 1, one.kps};
     }
     if (!table_ok) return {t64 <= 2 * cus ? SMALL_64x64 : SMALL_128x64, 1, one.kps};
