@@ -1633,12 +1633,12 @@ float *scratch_ptr() {
 // with late fold operands, and with how many K ranges per workgroup; tile -1: the tile table.
 // A call that asks for no split (splits = 1) is one chain of 16-k blocks per output in the direct-to-LDS order whatever kernel it
 // gets here, and the table's for K >= 64, so its bits depend neither on M nor on the epilogue nor (K % 64 == 0, or unaligned) on the
-// weight's layout; the ranges serve calls that leave the split to the library (splits = 0).
+// weight's layout; the ranges serve calls that leave the split to the library (splits = 0), there too the same for W and W^T.
 // The lines were measured on MI355X in replayed graphs (us; fold / stats: with the LayerNorm fold from row partials / bias, residual,
 // row partials).
 // One chain:
 //  - up to two 64 x 64 tiles per CU: that tile (256 x 768 x 3072 12.4 against 13.2 for the table, with stats 13.2 against 23.8;
-//    fold 588 x 2304 x 768 8.9 against 11.0; 1024 x 2304 (576 tiles): level).
+//    fold 588 x 2304 x 768 8.9 against 11.0; W^T 588 x 768 x 768 5.2 against 5.8, x 3072 14.5 against 16.8; 1024 x 2304 (576 tiles): level).
 //    With the fold on at most one 32 x 32 tile per CU that tile, a wavefront each (256 x 768 x 768 6.3 against 6.8).
 //  - 16-byte operands with K % 64 != 0: W always the table (50 x 2048 x 720 5.8 against 6.7, 256 x 768 x 3080 16.2 against 16.4), W^T
 //    below K = 384 (64 x 512 x 136 3.6 against 4.2, 1000 x 504 x 328 5.1 against 5.4; 50 x 720 x 720 7.3 against 6.5).
@@ -1683,8 +1683,8 @@ SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats,
         const SplitK sk = ranges(4);
         if (force == SMALL_RANGES_32 || (force == SMALL_RANGES_64 && !ln)) return {force, sk.splits, sk.kps};
         if ((force == SMALL_64x64 || force == SMALL_128x64) && !ln && !stats && r.ldx >= 8 && r.ldw >= 8) return {force, 1, one.kps};
-        if (force == SMALL_DMA && fast && !r.wt) return {force, 1, one.kps};
-        if (force == SMALL_DMA2 && fast && !r.wt && r.K % 128 == 0 && r.splits == 0) return {force, 1, r.K / 2};
+        if (force == SMALL_DMA && fast) return {force, 1, one.kps};
+        if (force == SMALL_DMA2 && fast && r.K % 128 == 0 && r.splits == 0) return {force, 1, r.K / 2};
         return none;
     }
     if (any && vec && t64 <= 2 * cus && (r.wt ? r.K < 384 : r.K < 512 || r.splits != 0)) return none;
@@ -1696,7 +1696,7 @@ SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats,
         const SplitK sk = ranges(kSmallMaxRanges64);
         return {SMALL_RANGES_64, sk.splits, sk.kps};
     }
-    if (fast && !r.wt) {
+    if (fast) {
         if (t64 <= cus && r.K >= 1024 && r.K % 128 == 0 && r.splits == 0) return {SMALL_DMA2, 1, r.K / 2};
         if (t64 <= 2 * cus) return {SMALL_DMA, 1, one.kps};
     }
@@ -1706,8 +1706,10 @@ SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats,
 
 // The 64 x 64 direct-to-LDS tile of small problems (LATE builds of k_gemm5), one or two K ranges per workgroup.
 struct SmallDma { KernelFn fn; uint32_t threads; size_t lds; bool attr_set; };
-SmallDma g_small_dma[2] = {{k_gemm5<64, 64, 64, 3, false, 2, false, true, 1, EPI_ANY, true>, 256, Cfg5<64, 64, 64, 3, false>::LDS, false},
-                           {k_gemm5<64, 64, 64, 3, false, 1, false, true, 2, EPI_ANY, true>, 512, 2 * Cfg5<64, 64, 64, 3, false>::LDS, false}};
+SmallDma g_small_dma[2][2] = {{{k_gemm5<64, 64, 64, 3, false, 2, false, true, 1, EPI_ANY, true>, 256, Cfg5<64, 64, 64, 3, false>::LDS, false},
+                              {k_gemm5<64, 64, 64, 3, false, 1, false, true, 2, EPI_ANY, true>, 512, 2 * Cfg5<64, 64, 64, 3, false>::LDS, false}},
+                             {{k_gemm5<64, 64, 64, 3, true, 2, false, true, 1, EPI_ANY, true>, 256, Cfg5<64, 64, 64, 3, true>::LDS, false},
+                              {k_gemm5<64, 64, 64, 3, true, 1, false, true, 2, EPI_ANY, true>, 512, 2 * Cfg5<64, 64, 64, 3, true>::LDS, false}}};
 template <typename SetEpi>
 int launch_small(const GemmReq &r, const SmallPlan &sp, bool any, SetEpi set_epi, const char *name) {
     const sh_gemm_epi *e = r.epi;
@@ -1722,7 +1724,7 @@ int launch_small(const GemmReq &r, const SmallPlan &sp, bool any, SetEpi set_epi
         sh_cdiv(std::min(r.M, r.N), 32) > 65535) { sh_set_error(-1, "[%s] problem too large", name); return -1; }
     a.tiles_m = sh_cdiv(r.M, kSmallDims[sp.tile].bm); a.tiles_n = sh_cdiv(r.N, kSmallDims[sp.tile].bn);
     if (sp.tile >= SMALL_ANY_TILES) {
-        SmallDma &d = g_small_dma[sp.tile - SMALL_DMA];
+        SmallDma &d = g_small_dma[r.wt][sp.tile - SMALL_DMA];
         if (!d.attr_set) { (void)hipFuncSetAttribute((const void *)d.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)d.lds); d.attr_set = true; }
         const uint32_t nblk = grid_of(a);
         hipLaunchKernelGGL(d.fn, dim3(nblk), dim3(d.threads), d.lds, sh_stream(), a);

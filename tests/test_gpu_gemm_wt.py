@@ -116,3 +116,21 @@ def test_wt_encoder_shapes_match_natural_layout(lib, gpu, N, K, epi):
         want = want + r[rows].astype(np.float32)
     bad, err, _ = refs.close(to_np(Z)[rows], want)
     assert bad == 0, err
+
+
+@pytest.mark.parametrize("splits", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(512, 1536, 1024), (256, 3072, 1024), (1024, 768, 3072), (588, 768, 3072), (512, 1536, 960), (256, 2560, 960),
+                                   (588, 2304, 768), (256, 768, 3072), (50, 720, 768), (147, 64, 128), (4096, 1024, 768), (100, 100, 588), (300, 717, 301)])
+def test_wt_small_problems_match_natural_layout(lib, gpu, M, N, K, splits):
+    """Problems of few tiles (one and two K ranges of the 64 x 64 tile, ranges of a wavefront each) and unaligned operands:
+    W^T and W take the same ranges, whether the split is none or the library's choice."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(6)
+    X = torch.randn(M, K, generator=g, device="cuda").half()
+    W = (torch.randn(K, N, generator=g, device="cuda") * K ** -0.5).half()
+    WT, R = W.t().contiguous(), torch.randn(M, N, generator=g, device="cuda").half()
+    for e in (shops.epi(splits=splits), shops.epi(residual=A(R), ldr=N, splits=splits)):
+        z = [torch.empty(M, N, device="cuda", dtype=torch.float16) for _ in range(2)]
+        assert lib.sh_gemm_ex(A(X), A(W), A(z[0]), M, N, K, K, N, N, None, e) == 0, shops.last_error()
+        assert lib.sh_gemm_ex_wt(A(X), A(WT), A(z[1]), M, N, K, K, K, N, None, e) == 0, shops.last_error()
+        assert np.array_equal(codes(z[0]), codes(z[1]))
