@@ -1656,7 +1656,7 @@ struct SmallPlan { int tile; uint32_t ranges, kps; };
 SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats, bool ln_reg) {
     const SmallPlan none{-1, 0, 0};
     const int force = env_int("SH_GEMM_SMALL", -1);      // tests: -2 = the table, >= 0 = that variant where it can run
-    if (force == -2 || r.K == 0 || env_int("SH_GEMM_CFG", -1) >= 0) return none;
+    if (force == -2 || r.K == 0 || env_int("SH_GEMM_CFG", -1) >= 0 || (r.splits == 0 && env_int("SH_GEMM_SPLITS", 0) > 0)) return none;
     if ((ln && !ln_reg) || r.ldx >= (1u << 23) || r.ldw >= (1u << 23)) return none;
     const uint32_t wr = r.wt ? r.N : r.K, wc = r.wt ? r.K : r.N;
     const bool any = !vec || !fast;                      // needs the any-alignment build

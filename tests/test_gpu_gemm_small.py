@@ -136,3 +136,18 @@ def test_an_unsplit_product_is_one_chain(lib, gpu, N, K, off):
             Z = torch.empty(m, N, device="cuda", dtype=torch.float16)
             assert lib.sh_gemm_ex(A(xb), A(W), A(Z), m, N, K, K, N, N, cfg, e) == 0, (name, shops.last_error())
             assert np.array_equal(to_np(Z), z[:m]), (name, m)          # (values: -0 + 0 is +0)
+
+
+def test_a_forced_split_count_reaches_small_problems(lib, gpu, monkeypatch):
+    """SH_GEMM_SPLITS sets the split of a call that leaves it to the library: the bits of the same request."""
+    import torch
+    M, N, K = 256, 512, 1536
+    X, W = to_dev(data.normal((M, K), 21)), to_dev(data.normal((K, N), 22, std=1 / np.sqrt(K)))
+    z = {}
+    for name, splits, env in (("asked", 3, None), ("forced", 0, "3"), ("free", 0, None)):
+        monkeypatch.setenv("SH_GEMM_SPLITS", env) if env else monkeypatch.delenv("SH_GEMM_SPLITS", raising=False)
+        Z = torch.empty(M, N, device="cuda", dtype=torch.float16)
+        assert lib.sh_gemm_ex(A(X), A(W), A(Z), M, N, K, K, N, N, None, shops.epi(splits=splits)) == 0, shops.last_error()
+        z[name] = codes(Z)
+    assert np.array_equal(z["asked"], z["forced"])
+    assert not np.array_equal(z["free"], z["forced"])                  # (four or eight ranges without it)
