@@ -1648,6 +1648,9 @@ float *scratch_ptr() {
 //    tile per CU they lose (588 x 768: 6.1 against 5.6).
 //  - up to one 64 x 32 tile per CU with a long K: the same with 64-row tiles.
 //  - up to one 64 x 64 tile per CU from K = 1024 on: that tile with two ranges (1024 x 768 x 3072 with stats: 13.4 against 15.9).
+//  - past K = 4096 the table's split-K, whose ranges run on more workgroups, takes over (64 x 64 x 8192 7.9 against 12.0, x 65536 20.7
+//    against 113.6, 512 x 768 x 8192 18.7 against 24.4; 256 x 1024 x 4096 11.1 against 9.8). Unaligned operands keep the ranges
+//    (50 x 721 x 16393: 52.7 against 100.9).
 //  - 16-byte operands whose K is no multiple of 64: the table below K = 512 (64 x 512 x 136 3.9 against 4.6, x 456 level), for W^T
 //    below 384, up to two 64 x 64 tiles per CU (4096 x 768 x 328 12.0 against 11.0).
 // Operands without 16-byte alignment, and other W^T with K % 64 != 0: never the table, whose element-wise kernels are 4 to
@@ -1688,6 +1691,7 @@ SmallPlan small_plan(const GemmReq &r, bool vec, bool fast, bool ln, bool stats,
         return none;
     }
     if (any && vec && t64 <= 2 * cus && (r.wt ? r.K < 384 : r.K < 512 || r.splits != 0)) return none;
+    if (r.splits == 0 && r.K > 4096 && t64 <= 2 * cus && vec) return none;
     if (t32 <= cus && (r.splits == 0 || !fast || ln)) {
         const SplitK sk = ranges(4 * t32 <= cus ? kSmallMaxRanges : kSmallMaxRanges / 2);
         return {SMALL_RANGES_32, sk.splits, sk.kps};
