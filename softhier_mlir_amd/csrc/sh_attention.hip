@@ -885,24 +885,24 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
     attn_stamp(stamp, last, 6);
 }
 
-// Attention of few workgroups (one or a few short sequences, and every token-masked head): a workgroup owns 32 queries of
-// one head and its wavefronts split the key blocks (wavefront w takes blocks w, w + W, ...), each with a running maximum, row
-// sum and O of its own, combined through LDS at the end. k_flash3's 128 queries per workgroup make 24 workgroups of one S = 256
-// sequence of 12 heads, each a chain of four key blocks (6.5 us, and 33 us with the token mask of the two-pass kernel,
-// whose 64 token reads per lane went to memory one by one); here they are 96 workgroups of one block per wavefront.
-// Latency bounds it: K fragments come straight from global memory into registers (each block's K, V and token loads are
-// all in flight together, the next block's issued before the exponentials), V goes through the wavefront's own LDS stage for the transpose
-// reads, and no barrier is crossed before the combine. p = 2^(c s - m) with the scores in fp32, so any scale and sign.
-// MASK: key j is allowed for query i iff tok[j] <= tok[i]; a padding query, or one whose allowed keys all score -inf, averages
+// Token-masked heads (S <= 256, S % 4 == 0): a workgroup owns 32 queries of one head and wavefront w its key block w (up to
+// four), with a maximum, row sum and O of its own, combined through LDS at the end. 128 queries per workgroup make 30 workgroups
+// of one S = 256 sequence of 15 heads, each a chain of four key blocks (34.6 us in a two-pass kernel whose 64 token reads per
+// lane went to memory one by one); here they are 120 workgroups of one block per wavefront, 6.6 us.
+// Latency bounds it: K fragments come straight from global memory into registers (the block's K, V and token loads are all in
+// flight together), V goes through the wavefront's own LDS stage for the transpose reads, and no barrier is crossed before the
+// combine. p = 2^(c s - m) with the scores in fp32, so any scale and sign.
+// (Unmasked heads of few workgroups gained little from it, B = 1, S = 256, 12 heads 5.9 against k_flash3's 6.3, B = 1, S = 1024, 4 heads
+// 10.8 against 13.3, and stored other bits than k_flash3: a sequence's output then depended on what it was batched with.)
+// Key j is allowed for query i iff tok[j] <= tok[i]; a padding query, or one whose allowed keys all score -inf, averages
 // V uniformly over the S keys.
-// Masked heads of 32 / 72 / 80 / 96 (P2) hold each numerator as two fp16 halves of 2^15 p, 22 bits down to 2^-29, and sum them
+// Heads of 32 / 72 / 80 / 96 (P2) hold each numerator as two fp16 halves of 2^15 p, 22 bits down to 2^-29, and sum them
 // unrounded: the per-query kernel they would take otherwise keeps p in fp32, and one fp16 half loses a tail below 2^-25 of the maximum.
-// Workgroups past the (query block, head, sequence) items read the caller's prefetch ranges (a.pf0, a.pf1).
 typedef uint32_t attn_u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t attn_u4 __attribute__((ext_vector_type(4)));
 typedef attn_u2 attn_u2_a2 __attribute__((aligned(2)));      // four tokens, 2-byte aligned
-template <int DH, bool MASK>
-__global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a, ShDiv dgx, ShDiv dh_, uint32_t items, uint64_t *stamp) {
+template <int DH>
+__global__ __launch_bounds__(256) void k_flash_split(AttnArgs a, ShDiv dgx, ShDiv dh_, uint64_t *stamp) {
     constexpr int DC = DH / 8, NS = (DC + 1) / 2, DT = (DH + 31) / 32;
     constexpr int VCH = KB * DC;                     // 16-byte chunks of a V block
     constexpr int OP = DH + 4;                       // fp32 pitch of a query's O row in the combine (conflict-free writes)
@@ -910,21 +910,12 @@ __global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a
     extern __shared__ uint4 smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = (int)(blockDim.x >> 6);
     const int g = lane >> 5, r32 = lane & 31, q4 = lane >> 4, iq = lane & 15;
-    if (blockIdx.x >= items) {                       // prefetch workgroups: one load per 64-byte line, nothing kept
-        const uint64_t n = (uint64_t)a.pfl0 + a.pfl1;
-        for (uint64_t j = (uint64_t)(blockIdx.x - items) * blockDim.x + threadIdx.x; j < n; j += (uint64_t)(gridDim.x - items) * blockDim.x) {
-            const uint8_t *p = j < a.pfl0 ? a.pf0 + j * 64 : a.pf1 + (j - a.pfl0) * 64;
-            const uint32_t v = *(const uint32_t *)p;
-            asm volatile("" ::"v"(v));
-        }
-        return;
-    }
     const uint32_t hb = sh_div(blockIdx.x, dgx), qb = blockIdx.x - hb * dgx.d, b = sh_div(hb, dh_), h = hb - b * dh_.d;
-    const uint32_t S = a.S, nkb = (S + KB - 1) / KB, q0 = qb * 32, myq = q0 + r32;
+    const uint32_t S = a.S, k0 = wave * KB, q0 = qb * 32, myq = q0 + r32;
     const uint16_t *Q = a.q + b * a.bsq + (uint64_t)h * DH;
     const uint16_t *Kp = a.k + b * a.bsk + (uint64_t)(h / a.grp) * DH;
     const uint16_t *Vp = a.v + b * a.bsv + (uint64_t)(h / a.grp) * DH;
-    const bool last = stamp && threadIdx.x == 0 && blockIdx.x == items - 1;
+    const bool last = stamp && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1;
     attn_stamp(stamp, stamp && threadIdx.x == 0 && blockIdx.x == 0, 7);
     attn_stamp(stamp, last, 0);
 
@@ -932,124 +923,108 @@ __global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a
     const uint32_t lds0 = sh_lds_addr(mine);
     // K fragment (tt, s) of a block: key 32 tt + r32, dh 16 s + 8 g (zero past DH); V: chunk lane + 64 i of the block
     attn_u4 kr[2][NS], vr[DC];
-    attn_u2 tr[MASK ? 2 : 1][MASK ? 4 : 1];          // tokens of the lane's keys: 32 tt + 8 e + 4 g ..+3
-    auto load = [&](uint32_t kb) __attribute__((always_inline)) {
-        const uint32_t k0 = kb * KB;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const uint16_t *p = Kp + (uint64_t)min(k0 + 32 * tt + r32, S - 1) * a.ldk;
-#pragma unroll
-            for (int s = 0; s < NS; ++s) kr[tt][s] = *(const attn_u4 *)(p + ((DC & 1) && s == NS - 1 ? 16 * s : 16 * s + 8 * g));
-        }
-#pragma unroll
-        for (int i = 0; i < DC; ++i) {
-            const uint32_t c = lane + 64 * i, key = c / DC, pc = c % DC;
-            vr[i] = *(const attn_u4 *)(Vp + (uint64_t)min(k0 + key, S - 1) * a.ldv + 8 * pc);
-        }
-        if constexpr (MASK) {                        // (S % 4 == 0: a group of four keys is whole or past S)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) tr[tt][e] = *(const attn_u2_a2 *)(a.tok + min(k0 + 32 * tt + 8 * e + 4 * g, S - 4));
-        }
-    };
-    const uint32_t tq = MASK ? (uint32_t)a.tok[min(myq, S - 1)] : 0u;
+    attn_u2 tr[2][4];                                // tokens of the lane's keys: 32 tt + 8 e + 4 g ..+3
+    const uint32_t tq = (uint32_t)a.tok[min(myq, S - 1)];
     attn_u4 qr[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s)
         qr[s] = *(const attn_u4 *)(Q + (uint64_t)min(myq, S - 1) * a.ldq + ((DC & 1) && s == NS - 1 ? 16 * s : 16 * s + 8 * g));
-    load(min((uint32_t)wave, nkb - 1));
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+        const uint16_t *p = Kp + (uint64_t)min(k0 + 32 * tt + r32, S - 1) * a.ldk;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) kr[tt][s] = *(const attn_u4 *)(p + ((DC & 1) && s == NS - 1 ? 16 * s : 16 * s + 8 * g));
+    }
+#pragma unroll
+    for (int i = 0; i < DC; ++i) {
+        const uint32_t c = lane + 64 * i, key = c / DC, pc = c % DC;
+        vr[i] = *(const attn_u4 *)(Vp + (uint64_t)min(k0 + key, S - 1) * a.ldv + 8 * pc);
+    }
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)                   // (S % 4 == 0: a group of four keys is whole or past S)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tr[tt][e] = *(const attn_u2_a2 *)(a.tok + min(k0 + 32 * tt + 8 * e + 4 * g, S - 4));
     attn_stamp(stamp, last, 1);
     attn_stamp(stamp, last, 2);
     sh_h8 qf[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) qf[s] = (DC & 1) && s == NS - 1 && g == 1 ? sh_h8{} : __builtin_bit_cast(sh_h8, qr[s]);
-    const bool uni = MASK && tq == kLlmPad;
+    const bool uni = tq == kLlmPad;
     const float c = a.c;
-    constexpr bool P2 = MASK && DH != 64 && DH != 128;
+    constexpr bool P2 = DH != 64 && DH != 128;
     const sh_h2 one2 = {(_Float16)1.0f, (_Float16)1.0f};
     sh_f16v oacc[DT];
 #pragma unroll
     for (int i = 0; i < DT; ++i) oacc[i] = sh_f16v{};
-    float m = -INFINITY, l = 0.f;
-
-    for (uint32_t kb = wave; kb < nkb; kb += W) {
-        sh_f16v sacc[2];
+    sh_f16v sacc[2];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            sacc[tt] = sh_f16v{};
+    for (int tt = 0; tt < 2; ++tt) {
+        sacc[tt] = sh_f16v{};
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                const sh_h8 kf = (DC & 1) && s == NS - 1 && g == 1 ? sh_h8{} : __builtin_bit_cast(sh_h8, kr[tt][s]);
-                sacc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[s], sacc[tt], 0, 0, 0);
-            }
+        for (int s = 0; s < NS; ++s) {
+            const sh_h8 kf = (DC & 1) && s == NS - 1 && g == 1 ? sh_h8{} : __builtin_bit_cast(sh_h8, kr[tt][s]);
+            sacc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[s], sacc[tt], 0, 0, 0);
         }
-        asm volatile("" ::: "memory");               // (one wavefront's LDS instructions execute in order)
-#pragma unroll
-        for (int i = 0; i < DC; ++i) {
-            const uint32_t ci = lane + 64 * i, key = ci / DC, pc = ci % DC;
-            *(attn_u4 *)(mine + (key * DC + (DH == 64 || DH == 128 ? pc ^ vfw<DH>(key) : pc)) * 16) = vr[i];
-        }
-        // t = c s, -inf for keys without weight; a padding query's keys all weigh the same
-        const bool tail = (kb + 1) * KB > S;
-        float mb = -INFINITY;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float t = sacc[tt][r] * c;
-                if constexpr (MASK) {
-                    const uint32_t w = (r & 2) ? tr[tt][r >> 2].y : tr[tt][r >> 2].x, tk = (r & 1) ? w >> 16 : w & 0xFFFFu;
-                    t = uni ? 0.f : tk <= tq ? t : -INFINITY;
-                }
-                if (tail && kb * KB + 32 * tt + 8 * (r >> 2) + 4 * g + (r & 3) >= S) t = -INFINITY;
-                sacc[tt][r] = t;
-                mb = fmaxf(mb, t);
-            }
-        if (kb + W < nkb) load(kb + W);              // into the registers just read: in flight during the exponentials and P.V
-        mb = sh_max_xor32(mb);
-        const float mn = fmaxf(m, mb), ms = mn == -INFINITY ? 0.f : mn, alpha = sh_fast_exp2(m - ms);
-        m = mn;
-        sh_h8 pf[4], pl[P2 ? 4 : 1];
-        l *= alpha;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float p = sh_fast_exp2(sacc[tt][r] - ms) * (P2 ? 32768.f : 1.f);
-                const _Float16 hi = (_Float16)p;
-                pf[2 * tt + (r >> 3)][r & 7] = hi;
-                if constexpr (P2) {
-                    pl[2 * tt + (r >> 3)][r & 7] = (_Float16)(p - (float)hi);
-                    l += p;
-                }
-            }
-#pragma unroll
-        for (int sp = 0; sp < (P2 ? 0 : 4); ++sp) {
-            const uint4 w = __builtin_bit_cast(uint4, pf[sp]);
-            l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.x), one2, l, false);
-            l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.y), one2, l, false);
-            l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.z), one2, l, false);
-            l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.w), one2, l, false);
-        }
-#pragma unroll
-        for (int i = 0; i < DT; ++i) oacc[i] *= alpha;
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int sp = 0; sp < 4; ++sp)
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {        // (columns past DH read the next rows or the 64 bytes behind the block: outputs that are not stored)
-                const uint32_t d = 32 * dt + 16 * (q4 & 1) + 4 * (iq & 3), k0 = 16 * sp + 4 * g + (iq >> 2);
-                const uint32_t ch = DH == 64 || DH == 128 ? (d >> 3) ^ vfw<DH>(k0) : d >> 3;
-                const uint32_t at = lds0 + k0 * (DH * 2) + 16 * ch + 2 * (d & 7);
-                const sh_s4 lo = sh_ds_read_tr(at), hi = sh_ds_read_tr(at + 8 * (DH * 2));
-                const sh_h8 vf = __builtin_bit_cast(sh_h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[sp], oacc[dt], 0, 0, 0);
-                if constexpr (P2) oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[sp], oacc[dt], 0, 0, 0);
-            }
-        asm volatile("" ::: "memory");
-        if (kb == (uint32_t)wave) { attn_stamp(stamp, last, 3); attn_stamp(stamp, last, 4); }
     }
+    asm volatile("" ::: "memory");               // (one wavefront's LDS instructions execute in order)
+#pragma unroll
+    for (int i = 0; i < DC; ++i) {
+        const uint32_t ci = lane + 64 * i, key = ci / DC, pc = ci % DC;
+        *(attn_u4 *)(mine + (key * DC + (DH == 64 || DH == 128 ? pc ^ vfw<DH>(key) : pc)) * 16) = vr[i];
+    }
+    // t = c s, -inf for keys without weight; a padding query's keys all weigh the same
+    const bool tail = k0 + KB > S;
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float t = sacc[tt][r] * c;
+            const uint32_t w = (r & 2) ? tr[tt][r >> 2].y : tr[tt][r >> 2].x, tk = (r & 1) ? w >> 16 : w & 0xFFFFu;
+            t = uni ? 0.f : tk <= tq ? t : -INFINITY;
+            if (tail && k0 + 32 * tt + 8 * (r >> 2) + 4 * g + (r & 3) >= S) t = -INFINITY;
+            sacc[tt][r] = t;
+            m = fmaxf(m, t);
+        }
+    m = sh_max_xor32(m);
+    const float ms = m == -INFINITY ? 0.f : m;
+    sh_h8 pf[4], pl[P2 ? 4 : 1];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float p = sh_fast_exp2(sacc[tt][r] - ms) * (P2 ? 32768.f : 1.f);
+            const _Float16 hi = (_Float16)p;
+            pf[2 * tt + (r >> 3)][r & 7] = hi;
+            if constexpr (P2) {
+                pl[2 * tt + (r >> 3)][r & 7] = (_Float16)(p - (float)hi);
+                l += p;
+            }
+        }
+#pragma unroll
+    for (int sp = 0; sp < (P2 ? 0 : 4); ++sp) {
+        const uint4 w = __builtin_bit_cast(uint4, pf[sp]);
+        l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.x), one2, l, false);
+        l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.y), one2, l, false);
+        l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.z), one2, l, false);
+        l = __builtin_amdgcn_fdot2(__builtin_bit_cast(sh_h2, w.w), one2, l, false);
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int sp = 0; sp < 4; ++sp)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {        // (columns past DH read the next rows or the 64 bytes behind the block: outputs that are not stored)
+            const uint32_t d = 32 * dt + 16 * (q4 & 1) + 4 * (iq & 3), vk = 16 * sp + 4 * g + (iq >> 2);
+            const uint32_t ch = DH == 64 || DH == 128 ? (d >> 3) ^ vfw<DH>(vk) : d >> 3;
+            const uint32_t at = lds0 + vk * (DH * 2) + 16 * ch + 2 * (d & 7);
+            const sh_s4 lo = sh_ds_read_tr(at), hi = sh_ds_read_tr(at + 8 * (DH * 2));
+            const sh_h8 vf = __builtin_bit_cast(sh_h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[sp], oacc[dt], 0, 0, 0);
+            if constexpr (P2) oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[sp], oacc[dt], 0, 0, 0);
+        }
+    asm volatile("" ::: "memory");
+    attn_stamp(stamp, last, 3);
+    attn_stamp(stamp, last, 4);
     attn_stamp(stamp, last, 5);
     // combine: each wavefront's O^T (lane (q, g): rows 32 dt + 8 (r / 4) + 4 g + r % 4 of query q), m and l of its 32 queries
     l += __shfl_xor(l, 32, 64);
@@ -1080,7 +1055,7 @@ __global__ __launch_bounds__(DH <= 64 ? 512 : 256) void k_flash_split(AttnArgs a
             o[0] = fmaf(f, lo.x, o[0]); o[1] = fmaf(f, lo.y, o[1]); o[2] = fmaf(f, lo.z, o[2]); o[3] = fmaf(f, lo.w, o[3]);
             o[4] = fmaf(f, hi.x, o[4]); o[5] = fmaf(f, hi.y, o[5]); o[6] = fmaf(f, hi.z, o[6]); o[7] = fmaf(f, hi.w, o[7]);
         }
-        if (MASK && mx == -INFINITY) {               // no key has weight
+        if (mx == -INFINITY) {               // no key has weight
             lt = (float)S;
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = 0.f;
@@ -1237,37 +1212,28 @@ int run(uint64_t q, uint64_t k, uint64_t v, uint64_t o, uint32_t B, uint32_t S, 
     static const int impl = [] { const char *e = getenv("SH_ATTN_IMPL"); return (e && *e) ? atoi(e) : 0; }();
     const dim3 grid(sh_cdiv(S, QPB), H, B);
     const bool fold = fabsf(a.c) <= 1.f;            // c q stays in fp16 range
-    // k_flash_split: every token-masked head it has a build for, and unmasked 64-wide heads while each of its wavefronts
-    // has a SIMD of its own and there are key blocks to share (graph replays, us, against k_flash3: B = 1, S = 256, 12 heads
-    // 5.9 / 6.3; B = 2 5.7 / 6.6; B = 3, S = 196 (1008 wavefronts) 6.8 / 7.6; B = 1, S = 1024, 4 heads (1024) 10.8 / 13.3;
-    // past that B = 4, S = 256 8.5 / 6.4; two key blocks, S = 128: 5.4 / 5.4)
-    auto split_fn = [&]() -> void (*)(AttnArgs, ShDiv, ShDiv, uint32_t, uint64_t *) {
+    const auto sfn = [&]() -> void (*)(AttnArgs, ShDiv, ShDiv, uint64_t *) {     // token-masked heads of the widths with a build
+        if (!tok || !vec || S > 4 * KB || S % 4) return nullptr;
         switch (dh) {
-            case 32: return tok ? k_flash_split<32, true> : nullptr;
-            case 64: return tok ? k_flash_split<64, true> : k_flash_split<64, false>;
-            case 72: return tok ? k_flash_split<72, true> : nullptr;
-            case 80: return tok ? k_flash_split<80, true> : nullptr;
-            case 96: return tok ? k_flash_split<96, true> : nullptr;
-            case 128: return tok ? k_flash_split<128, true> : nullptr;
+            case 32: return k_flash_split<32>;
+            case 64: return k_flash_split<64>;
+            case 72: return k_flash_split<72>;
+            case 80: return k_flash_split<80>;
+            case 96: return k_flash_split<96>;
+            case 128: return k_flash_split<128>;
             default: return nullptr;
         }
-    };
-    const uint64_t items = (uint64_t)sh_cdiv(S, 32) * H * B, simds = 4 * (uint64_t)(sh_num_cus() > 0 ? sh_num_cus() : 256);
-    const uint32_t waves = std::min<uint32_t>(sh_cdiv(S, KB), dh > 64 ? 4 : 8);
-    const auto sfn = vec && (tok || (impl == 0 && waves > 2 && items * waves <= simds)) && items < (1u << 30) ? split_fn() : nullptr;
+    }();
     if (sfn) {
-        const uint32_t pfb = (a.pfl0 | a.pfl1) ? (uint32_t)std::min<uint64_t>(256, ((uint64_t)a.pfl0 + a.pfl1 + 64 * waves - 1) / (64 * waves)) : 0u;
-        const uint32_t lds = waves * split_region(dh);
-        static bool attr_done[2][2];                 // (eight wavefronts of a 64-wide head, four of a 128-wide one)
-        if (lds > 64 * 1024 && !attr_done[dh > 64][tok != 0]) {
-            (void)hipFuncSetAttribute((const void *)sfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)((dh > 64 ? 4 : 8) * split_region(dh)));
-            attr_done[dh > 64][tok != 0] = true;
+        const uint32_t waves = sh_cdiv(S, KB), items = sh_cdiv(S, 32) * H * B, lds = waves * split_region(dh);
+        static bool attr_done = false;               // (four wavefronts of a 128-wide head)
+        if (lds > 64 * 1024 && !attr_done) {
+            (void)hipFuncSetAttribute((const void *)sfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(4 * split_region(dh)));
+            attr_done = true;
         }
-        const dim3 gr((uint32_t)items + pfb), bl(64 * waves);
         const ShDiv dx = sh_make_div(sh_cdiv(S, 32)), dhd = sh_make_div(H);
         g_prof.stamped = sp != nullptr;
-        hipLaunchKernelGGL(sfn, gr, bl, lds, st, a, dx, dhd, (uint32_t)items, sp);
-        a.pfl0 = a.pfl1 = 0;
+        hipLaunchKernelGGL(sfn, dim3(items), dim3(64 * waves), lds, st, a, dx, dhd, sp);
     } else if (tok) {
         if (S > 16384) { sh_set_error(-1, "[sh_attention] masked heads with dh=%u support S <= 16384", dh); return -1; }
         static bool attr_m = false;

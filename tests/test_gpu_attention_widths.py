@@ -1,7 +1,6 @@
 """Head widths and key-block splits of the attention kernels against the oracle: the one-pass kernel at every width it has a
-build for, on sequences that end inside, at and past a key block (64) and a query block (128), and the key-splitting kernel
-(short unmasked sequences of 64-wide heads, every token-masked head) at the edges of its 32-query items and of its
-wavefronts' key blocks."""
+build for, on sequences that end inside, at and past a key block (64) and a query block (128) and at few workgroups, and the
+key-splitting kernel of token-masked heads at the edges of its 32-query items and of its wavefronts' key blocks."""
 from __future__ import annotations
 
 import numpy as np
@@ -42,7 +41,7 @@ def test_one_pass_widths(lib, gpu, S, dh):
 
 @pytest.mark.parametrize("S,H", [(132, 3), (192, 4), (196, 12), (257, 2), (512, 2), (1000, 4)])
 @pytest.mark.parametrize("scale", [0.125, -0.3, 2.0])
-def test_split_keys_unmasked(lib, gpu, S, H, scale):
+def test_few_workgroups_unmasked(lib, gpu, S, H, scale):
     D = 64 * H
     q, k, v = (data.normal((S, D), 80 + i) for i in range(3))
     import torch

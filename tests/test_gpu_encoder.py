@@ -149,3 +149,20 @@ def test_captured_layer_survives_a_call_with_another_row_count(lib, gpu):
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
     del junk
+
+
+@pytest.mark.parametrize("sequence,S", [("fused", 196), ("fused", 256), ("reference", 256)])
+def test_a_sequence_does_not_depend_on_its_batch(lib, gpu, sequence, S):
+    """A sequence's output has the same bits alone and beside others: every GEMM of a layer is one chain per output whatever
+    kernel its row count takes, and attention is the same kernel at any number of workgroups."""
+    import torch
+    D, F, H = 768, 3072, 12
+    ps = [encoder.LayerParams.from_host(data.encoder_params(D, F, seed=400 + i)) for i in range(2)]
+    x = to_dev(data.normal((32 * S, D), 11))
+    outs = {}
+    for B in (1, 2, 3, 8, 32):
+        enc = encoder.Encoder(D, F, H)
+        outs[B] = enc.forward(x[:B * S].clone(), ps, B=B, S=S, sequence=sequence)
+    torch.cuda.synchronize()
+    for B, o in outs.items():
+        assert torch.equal(o.view(torch.int16), outs[32][:B * S].view(torch.int16)), B
