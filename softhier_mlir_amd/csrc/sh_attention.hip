@@ -1241,7 +1241,8 @@ int run(uint64_t q, uint64_t k, uint64_t v, uint64_t o, uint32_t B, uint32_t S, 
         go(k_attn_rows, dim3(S, H, B), S * sizeof(float));
     } else if ((dh == 32 || dh == 72 || dh == 80 || dh == 96) && vec &&
                (uint64_t)KB * (ldk > ldv ? ldk : ldv) * 2 < (1ull << 31)) {
-        // (these widths have the one build: no stamps, so the profile reports the launch's event time)
+        // (one build per width, so the widths between the powers of two that heads commonly have; 40, 48, 56, 88 and 104 to 120
+        // take the padded k_flash. No stamps: the profile reports the launch's event time)
         auto kern = dh == 32 ? k_flash3<32, 2, false, false, true, true> : dh == 72 ? k_flash3<72, 2, false, false, true, true>
                   : dh == 80 ? k_flash3<80, 2, false, false, true, true> : k_flash3<96, 2, false, false, true, true>;
         uint64_t *none = nullptr;

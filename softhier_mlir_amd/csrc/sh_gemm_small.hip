@@ -2,13 +2,17 @@
 // 16-byte alignment (sh_gemm.hip decides which calls come here: small_plan).
 //
 // What bounds such a product is latency: at M = 256 a 64 x 64 tiling of a 768-wide layer is 48 workgroups, each a chain
-// of k-slices that waits for memory two slices at a time. Here the chain is short-circuited by depth: R slices of 64 k
-// are in flight per workgroup in registers (plain 16-byte loads: one wavefront moves 25 B/clk with them, 11 with
+// of k-slices that waits for memory two slices at a time. Here R slices of 64 k per workgroup or wavefront are requested
+// ahead into registers (plain 16-byte loads: one wavefront moves 25 B/clk with them, 11 with
 // global -> LDS DMA, whose issue takes a wavefront ~90 cycles each; measured on resident data), tiles go down to 32 x 32
 // so that every CU has work, each slice is written to LDS once its loads have landed, and the fragments of slice kt are
 // read while the MFMAs of the one before run. The epilogue's operands are loaded before the k-loop.
+// As compiled, only the R = 4 build (64 x 64) keeps loads in flight through a wait (its waits stop at vmcnt 8). In the R = 2
+// builds the waits before the first of two slices' LDS writes go down to vmcnt 0 (14, 12, ... 0 for 32 x 32, 22 ... 0 for 64 x 32,
+// 5 ... 0 for 128 x 64), so both slices land together and a memory latency is exposed every 128 k.
 // The products are summed in the order of the direct-to-LDS kernels (16-k blocks in sequence through one MFMA chain per
-// output; with K ranges, the ranges' sums added in range order), so they store those kernels' bits.
+// output; with K ranges, which only a call with splits = 0 or two equal ranges gets, the ranges' sums added in range order), so
+// they store those kernels' bits.
 #include "sh_gemm_dev.h"
 #include "sh_gemm_small.h"
 #include <type_traits>
@@ -65,7 +69,6 @@ __global__ __launch_bounds__(KS && FM == 1 ? 512 : 256, KS ? 1 : 2) void k_gemm_
     const uint32_t kbeg = KS ? wave * a.kps : 0u, kend = KS ? min(a.K, kbeg + a.kps) : a.K;
     const int KT = kend > kbeg ? (int)((kend - kbeg + BK - 1) / BK) : 0;
     const uint32_t rem = EDGE && KT > 0 ? (kend - kbeg) - (uint32_t)(KT - 1) * BK : BK;     // (aligned: K % 64 == 0)
-    
 
     // Addresses: a wave-uniform base per operand and slice plus each lane's 32-bit byte offset of its chunk (the launch
     // checks the leading dims). xo / wo: any slice but the last; xl / wl: the last one, from a base 16 bytes lower, where a
@@ -117,8 +120,8 @@ __global__ __launch_bounds__(KS && FM == 1 ? 512 : 256, KS ? 1 : 2) void k_gemm_
         else wo[r] = (__umul24(c / WCPR, (uint32_t)a.ldw) + min(n0 + 8 * (c % WCPR), EDGE ? a.N - 1 : a.N - 8) - n0) * 2;
         wl[r] = EDGE ? last_w(r, sh, nv) : wo[r];
     }
-    // Slice kt into register set u. Always the same number of loads, so each wait counts exactly the loads behind it: a
-    // slice past the end re-reads the last one (a few cached lines).
+    // Slice kt into register set u. Always the same number of loads: a slice past the end re-reads the last one (a few
+    // cached lines).
     uint4 rx[R][XR], rw[R][WR];
     auto gload = [&](int kt, auto uc) __attribute__((always_inline)) {
         constexpr int u = decltype(uc)::value;
