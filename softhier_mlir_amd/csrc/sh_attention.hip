@@ -530,8 +530,8 @@ __global__ __launch_bounds__(256, DH == 64 ? 3 : 2) void k_flash2(AttnArgs a, ui
 constexpr float kTau = 8.f;
 // EX (widths 32 / 72 / 80 / 96): k_flash's arithmetic on this kernel's loads: the queries stay as given, m is the running maximum
 // itself and c s - m one fp32 multiply-add per score, so any scale will do and the bits are k_flash's. Against k_flash, padded
-// to 64 or 128: B = 4, S = 580, 16 heads of 80 64.8 -> 22.6 us, B = 1, S = 1024, 16 heads of 32 33.4 -> 13.3. (m left at 0 while the
-// first maximum was within kTau of it took 20.0 and 12.4 us, but numerators up to 2^8 smaller are lost to fp16 sooner: error against
+// to 64 or 128: B = 4, S = 580, 16 heads of 80 64.8 -> 21.6 us, B = 1, S = 1024, 16 heads of 32 33.4 -> 13.3. (m left at 0 while the
+// first maximum was within kTau of it took 19.0 and 12.4 us, but numerators up to 2^8 smaller are lost to fp16 sooner: error against
 // float64 2.93e-4 instead of 2.74e-4 on the first of these, 1.4e-2 for a long tail 17 units below its maximum.)
 template <int DH, int NST, bool PF = false, bool ST = true, bool RAG = true, bool EX = false>
 __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, uint64_t *stamp) {
@@ -888,7 +888,7 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void k_flash3(AttnArgs a, ui
 // Token-masked heads (S <= 256, S % 4 == 0): a workgroup owns 32 queries of one head and wavefront w its key block w (up to
 // four), with a maximum, row sum and O of its own, combined through LDS at the end. 128 queries per workgroup make 30 workgroups
 // of one S = 256 sequence of 15 heads, each a chain of four key blocks (34.6 us in a two-pass kernel whose 64 token reads per
-// lane went to memory one by one); here they are 120 workgroups of one block per wavefront, 6.6 us.
+// lane went to memory one by one); here they are 120 workgroups of one block per wavefront, 6.3 us.
 // Latency bounds it: K fragments come straight from global memory into registers (the block's K, V and token loads are all in
 // flight together), V goes through the wavefront's own LDS stage for the transpose reads, and no barrier is crossed before the
 // combine. p = 2^(c s - m) with the scores in fp32, so any scale and sign.
